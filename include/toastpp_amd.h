@@ -165,7 +165,14 @@ int tmi_solver_set_linsolver(tmi_solver s, const char *name, double tol);
 int tmi_solver_set_precon(tmi_solver s, int precon);            /* SetPrecon */
 int tmi_solver_set_maxit(tmi_solver s, int maxit);              /* SetLinSolverMaxit; 0 = n+1 */
 int tmi_solver_set_mode(tmi_solver s, int mode);                /* TMI_MODE_* */
-/* Column tile of the block modes (RHS columns per Krylov block; 0 = auto) */
+/* Small blocks (n x columns x bytes per value up to 8.5 MB, 64 columns at
+ * most) are solved by one cooperative kernel that keeps the Krylov vectors in
+ * registers and LDS (no reference counterpart); larger ones by a launch
+ * sequence on column tiles.  Naming a detail of the launch sequence -- tile,
+ * rows per wave, SpMM variant, compaction, graphs -- selects it for every
+ * solve of the handle; the autotuner keeps whichever is faster.  Same method,
+ * recurrences and stopping tests; sums in another order.
+ * Column tile of the launch sequence (RHS columns per Krylov block; 0 = auto) */
 int tmi_solver_set_tile(tmi_solver s, int tile);
 /* Node order of the solver's private copy of the system (no reference
  * counterpart): TMI_ORDER_MORTON relabels the nodes along a Z-order curve of

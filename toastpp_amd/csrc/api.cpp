@@ -521,6 +521,7 @@ int tmi_solver_set_tile(tmi_solver h, int tile)
     TMI_CHECK(tile == 0 || tile == 1 || tile == 2 || tile == 4 || tile == 8 || tile == 16 || tile == 32 || tile == 64,
               TMI_ERR_INVALID_ARG, "tile must be 0 (auto) or a power of two <= 64");
     S(h).tile = tile;
+    S(h).launch_sequence = tile != 0;
     API_END
 }
 
@@ -566,6 +567,7 @@ int tmi_solver_set_rows_per_wave(tmi_solver h, int rows)
     API_BEGIN
     TMI_CHECK(rows >= 0 && rows <= 63, TMI_ERR_INVALID_ARG, "rows per wave must be 0 .. 63");
     S(h).rpw = rows;
+    S(h).launch_sequence = true;
     API_END
 }
 
@@ -577,6 +579,7 @@ int tmi_solver_set_spmm_variant(tmi_solver h, int variant)
               "(row blocks with shared gathers), 4 (row blocks, software-pipelined) or 5 (row blocks on the "
               "matrix cores)");
     S(h).spmm_variant = variant;
+    S(h).launch_sequence = true;
     API_END
 }
 
@@ -596,6 +599,7 @@ int tmi_solver_set_compaction(tmi_solver h, int min_width)
                   min_width == 16 || min_width == 32,
               TMI_ERR_INVALID_ARG, "compaction width must be 0 (off) or a power of two <= 32");
     S(h).compact_min = min_width;
+    S(h).launch_sequence = true;
     API_END
 }
 
@@ -888,6 +892,7 @@ int tmi_solver_set_graphs(tmi_solver h, int enable)
     API_BEGIN
     Solver &s = S(h);
     s.use_graphs = enable != 0;
+    s.launch_sequence = true;
     if (!s.use_graphs) s.ex.drop_graphs();
     API_END
 }

@@ -198,6 +198,9 @@ void launch_permute_vals(bool cplx, int nnz, const int *slot, const double *val6
 // FP32 values into the row-block SpMM's order: out[k] = in[slot[k]] (w floats each)
 void launch_gather_vals32(int nnz, int w, const int *slot, const float *in, float *out, hipStream_t st);
 void launch_gather_vals64(int nnz, int w, const int *slot, const double *in, double *out, hipStream_t st);
+// values into the slices of a resident layout: out[i] = in[slot[i]], 0 where
+// slot[i] < 0 (es bytes each: 4, 8 or 16)
+void launch_slice_vals(int es, int nent, const int *slot, const void *in, void *out, hipStream_t st);
 // tile of right-hand sides / solutions between the caller's [n][ld] layout
 // (reference node order) and the solver's [n][K] tile (solver node order):
 // gather dst[r][c] = src[perm[r]][q0 + c] for c < kc, 0 for kc <= c < K;

@@ -1,5 +1,8 @@
 // Device-resident finite-element mesh (Tri3 / Tet4) and its QM description.
 #pragma once
+#include <memory>
+#include <mutex>
+
 #include "common.hpp"
 
 namespace tmi {
@@ -17,6 +20,20 @@ struct QM {
     int nq = 0, nm = 0, nqm = 0;
     std::vector<double> Q, M;          // nq x dim, nm x dim
     std::vector<int> lptr, lidx;       // link list (CSR)
+};
+
+// Rows of a relabelled system dealt to nr ranks of the resident solve
+// (krylov_resident.hpp): rank r holds positions r0 .. r1-1, [n r / nr, n (r+1)
+// / nr), filled with its rows by falling length; slices of 8 positions hold
+// their entries interleaved, padded to a multiple of 4 per row.
+struct ResLayout {
+    int nu = 0;                        // most LDS rows (own + halo) of a rank
+    int nent = 0;                      // slice entries
+    DBuf<int> srow, node;              // per position: relabelled row, mesh node
+    DBuf<int> rslice, sofs;            // first slice of each rank; entry bounds of each slice
+    DBuf<int> hofs, halo;              // halo positions of each rank, ascending
+    DBuf<unsigned short> lcol;         // per entry: LDS row of its column
+    DBuf<int> gcol, slot;              // per entry: position of its column; CSR entry, -1 for padding
 };
 
 struct Mesh {
@@ -67,7 +84,15 @@ struct Mesh {
         // every block has fewer than 65536 coefficients)
         DBuf<unsigned> rb_word;
         bool rb_word_ok = false;
+        // resident solve: the rows by recursive bisection of their nodes
+        // (positions n r / nr .. n (r+1) / nr are rank r's rows), and the
+        // layouts of nr = 1, 2, 4 .. 256 ranks, each built on first use
+        DBuf<int> part;
+        std::unique_ptr<ResLayout> res[9];
     } order[3];
+    std::mutex res_mu;                 // guards the building of res[]
+    // null: too large for the builders' LDS
+    const ResLayout *res_layout(int kind, int nr, hipStream_t st);
 
     int geo_stride() const { return dim == 3 ? GEO3 : GEO2; }
     void setup(hipStream_t st);        // Mesh::Setup on the GPU

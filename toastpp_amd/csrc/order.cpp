@@ -226,6 +226,38 @@ static void row_block_unions(int n, const std::vector<int> &rp, const std::vecto
     }
 }
 
+// Recursive bisection of the rows of ranks lo .. hi-1 (positions n lo / nr
+// .. n hi / nr) at the ranks' middle, across the longest side of their
+// nodes' bounding box: compact parts with short boundaries.  The bounds of
+// fewer ranks are bounds of more, so one split into 256 serves every count.
+// (A range of the
+// clustered order would not do: its last rows are the ones no cluster took,
+// from all over the mesh.)
+static void split_ranks(int dim, int n, int nr, int lo, int hi, const double *x, const std::vector<int> &node,
+                        std::vector<int> &row)
+{
+    if (hi - lo < 2) return;
+    const int mid = (lo + hi) / 2;
+    const int a = (int)((long)n * lo / nr), m = (int)((long)n * mid / nr), b = (int)((long)n * hi / nr);
+    double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
+    for (int i = a; i < b; i++)
+        for (int d = 0; d < dim; d++) {
+            const double v = x[(size_t)node[row[i]] * dim + d];
+            mn[d] = std::min(mn[d], v);
+            mx[d] = std::max(mx[d], v);
+        }
+    int d = 0;
+    for (int k = 1; k < dim; k++)
+        if (mx[k] - mn[k] > mx[d] - mn[d]) d = k;
+    if (m > a && m < b)
+        std::nth_element(row.begin() + a, row.begin() + m, row.begin() + b, [&](int p, int q) {
+            const double u = x[(size_t)node[p] * dim + d], v = x[(size_t)node[q] * dim + d];
+            return u != v ? u < v : p < q;
+        });
+    split_ranks(dim, n, nr, lo, mid, x, node, row);
+    split_ranks(dim, n, nr, mid, hi, x, node, row);
+}
+
 const Mesh::NodeOrder &Mesh::build_order(int kind, hipStream_t st)
 {
     TMI_CHECK(kind == ORDER_NATURAL || kind == ORDER_MORTON || kind == ORDER_CLUSTER, TMI_ERR_INVALID_ARG,
@@ -261,6 +293,13 @@ const Mesh::NodeOrder &Mesh::build_order(int kind, hipStream_t st)
         prp[r + 1] = at;
     }
     order.perm.upload(perm.data(), n, st);
+    {   // rows in the order of the resident solve's ranks
+        std::vector<int> part(n);
+        std::iota(part.begin(), part.end(), 0);
+        split_ranks(dim, n, 256, 0, 256, h_nodes.data(), perm, part);
+        order.part.upload(part.data(), n, st);
+        TMI_HIP(hipStreamSynchronize(st));   // part goes out of scope
+    }
     // 4 trailing copies of nnz: the LDS-DMA SpMM stages row pointers in 16-byte chunks
     prp.insert(prp.end(), 4, prp[n]);
     order.rowptr.upload(prp.data(), n + 5, st);

@@ -1,0 +1,206 @@
+// Host side of the resident solve (krylov_resident.hpp): when it is taken,
+// how the columns are split over launches and teams, and the launch itself.
+#include <algorithm>
+#include <climits>
+#include <cmath>
+
+#include "krylov_resident.hpp"
+#include "solver.hpp"
+
+namespace tmi {
+
+// When and how a solve runs resident.  Against the launch sequence (us per
+// iteration, 1 launch each; COCG/PCG/BiCGSTAB on disks and cylinders):
+//   n 3,169 real x 16: 7.5 / 31       n 31,525 c64 x 2 (BiCGSTAB): 24 / 97
+//   n 19,441 c32 x 24: 26 / 38        n 31,525 c64 x 16: 27 / 59
+//   n 31,525 c32 x 8: 24 / 39         n 103,267 c32 x 8: 42 / 54
+//   n 31,525 c32 x 32 (BiCGSTAB): 74 / 76    n 31,525 c32 x 64: 73 / 72
+//   n 50,653 c32 x 64 (2 launches): 126 / 95
+// so it is taken for blocks of up to RES_MAX_BYTES, in one launch.
+static constexpr size_t RES_MAX_BYTES = 8500000;
+// Teams: one column per team keeps the reductions small and the ranks few
+// (n 19,441 x 24: 8 ranks 26 us, 32 ranks 28; n 31,525 c64 x 16: 16 ranks 27,
+// 32 ranks 34) but every team reads the matrix: beyond RES_MAX_ENTRIES
+// entries per iteration (n 103,267 x 8: 4 teams 53 us, 1 team 42) the columns
+// share as few teams as hold them.  Tiny systems run on single workgroups
+// without any exchange (n 817 x 4: 7.0 us, 4 ranks 9.4; n 3,169 x 16: 11.2).
+static constexpr long RES_MAX_ENTRIES = 8000000;
+static constexpr int RES_ONE_WG = 1500;
+
+Solver::ResPlan Solver::resident_plan(int nq, int md)
+{
+    ResPlan none;
+    const bool mixed = md == TMI_MODE_MIXED_BLOCK, bicg = !pcg();
+    const VKind vk = mixed ? vk32() : vk64();
+    const size_t sz = vbytes(vk);
+    const bool wide = vk == VK_C64;
+    if (launch_sequence || lsolver == TMI_LSOLVER_GMRES || nq < 1 || nq > 64) return none;
+    if ((size_t)mesh->n * nq * sz > RES_MAX_BYTES) return none;
+    int pow = 1;
+    while (pow < nq) pow *= 2;
+    int T = mesh->n <= RES_ONE_WG ? RES_WG : pow;
+    if ((long)T * mesh->nnz > RES_MAX_ENTRIES && T > 1 && T < RES_WG) T = std::max(1, pow / (wide ? 8 : RES_KC));
+    for (;; T /= 2) {
+        if (T < 1) return none;
+        const int nr = RES_WG / T;
+        int kc = 1;
+        while (kc * T < nq) kc *= 2;
+        const int cl = wide ? std::min(kc, 2) : (kc >= 4 ? 4 : 1), lpr = kc / cl;
+        if (kc > RES_KC || lpr > RES_LANES) return none;
+        const int rows = (mesh->n + nr - 1) / nr, need = (rows * lpr + RES_NT - 1) / RES_NT;
+        int E = 1;
+        while (E < need) E *= 2;
+        // instantiations (krylov_resident_*.hip)
+        const int emax = cl == 1 ? (wide && bicg ? 4 : 8) : (bicg ? 2 : 4);
+        if (E > emax) continue;   // fewer, longer teams
+        const ResLayout *l = mesh->res_layout(order_kind, nr, st);
+        if (!l || l->nu == INT_MAX) continue;
+        if ((((size_t)l->nu * kc * sz + 15) & ~(size_t)15) + res_lds_fixed(kc) > RES_LDS) continue;
+        ResPlan p;
+        p.K = nq;
+        p.nr = nr;
+        p.kc = kc;
+        p.cl = cl;
+        p.E = E;
+        return p;
+    }
+}
+
+size_t Solver::resident_fixed_bytes()
+{
+    return (RES_PART_WORDS + RES_TOT_WORDS) * sizeof(res_u64) + sizeof(ResColOut) * 64 + sizeof(double) * 64 + 8;
+}
+
+const void *Solver::sliced(OpKind k, const ResLayout &l, int nr)
+{
+    int lg = 0;
+    while ((1 << lg) < nr) lg++;
+    SliceOp &o = slice_op[k][lg];
+    const bool f32 = k == OPK_32 || k == OPK_P32 || k == OPK_MF32;
+    const void *src = k == OPK_32 ? (const void *)sval32.p : k == OPK_64 ? (const void *)sval64.p
+                    : k == OPK_P32 ? (const void *)pval32.p : k == OPK_P64 ? (const void *)pval64.p
+                    : k == OPK_MF32 ? (const void *)mfval32.p : (const void *)mfval64.p;
+    const size_t es = (f32 ? 4 : 8) * (cplx ? 2 : 1);
+    if (!o.valid) {
+        o.v.alloc((size_t)l.nent * es);
+        launch_slice_vals((int)es, l.nent, l.slot.p, src, o.v.p, st);
+        TMI_HIP(hipStreamSynchronize(st));   // other streams read it next
+        o.valid = true;
+    }
+    return o.v.p;
+}
+
+// Columns 0 .. nq-1 in cooperative launches of plan.K columns.  Returns the
+// number of columns above the tolerance, or -1 when a launch was refused or
+// gave up (the fields then hold initial guesses or finished columns, a valid
+// start for the launch sequence).
+int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld,
+                           tmi_colstat *stats, int md, const double *h_omega)
+{
+    hipStream_t st = e.st;
+    const int n = mesh->n;
+    const bool mixed = md == TMI_MODE_MIXED_BLOCK, mf = h_omega != nullptr;
+    const bool cg = pcg(), bil = lsolver == TMI_LSOLVER_COCG, diag = precon == TMI_PRECON_DIAG;
+    const VKind vk = mixed ? vk32() : vk64();
+    const size_t sin = vbytes(vk), s64 = vbytes(vk64());
+    const int cap = (mixed && mixed_maxit > 0) ? mixed_maxit : (maxit > 0 ? maxit : n + 1);
+    const ResLayout &l = *mesh->res_layout(order_kind, plan.nr, this->st);   // built by the plan
+    ResArgs a{};
+    a.n = n;
+    a.kc = plan.kc;
+    a.nr = plan.nr;
+    a.maxit = cap;
+    a.ru = mixed ? reliable_every : (1 << 30);
+    a.mixed = mixed ? 1 : 0;
+    a.nu = l.nu;
+    a.tol2 = tol * tol;
+    // the recursive residual aims a little below the target so that the
+    // verifying FP64 residual usually passes at the first check
+    a.itol2 = mixed ? 0.25 * a.tol2 : a.tol2;
+    a.srow = l.srow.p;
+    a.node = l.node.p;
+    a.sofs = l.sofs.p;
+    a.rslice = l.rslice.p;
+    a.hofs = l.hofs.p;
+    a.halo = l.halo.p;
+    a.lcol = l.lcol.p;
+    a.gcol = l.gcol.p;
+    {
+        std::lock_guard<std::mutex> lk(prep_mu);
+        const bool right = diag && !cg;   // BiCGSTAB iterates with K D^-1
+        a.op = sliced(mf ? (mixed ? OPK_MF32 : OPK_MF64)
+                         : right ? (mixed ? OPK_P32 : OPK_P64) : (mixed ? OPK_32 : OPK_64), l, plan.nr);
+        a.op64 = (const double *)sliced(mf ? OPK_MF64 : OPK_64, l, plan.nr);
+    }
+    if (diag) {
+        if (mf) a.idiag = mixed ? (const void *)mfdiag32.p : (const void *)mfdiag64.p;
+        else a.idiag = mixed ? (const void *)idiag32.p : (const void *)idiag64.p;
+    }
+    a.b = d_b;
+    a.x = d_x;
+    a.ld = ld;
+    Exec::Resident &r = e.res;
+    const int teams = (plan.K + plan.kc - 1) / plan.kc;
+    const size_t elems = (size_t)n * teams * plan.kc;
+    if (r.pub_p.n < elems * sin) r.pub_p.alloc(elems * sin);
+    if (!cg && r.pub_s.n < elems * sin) r.pub_s.alloc(elems * sin);
+    if (!cg && !mixed && r.rd0.n < elems * sin) r.rd0.alloc(elems * sin);
+    if (r.x64.n < elems * s64) r.x64.alloc(elems * s64);
+    if (!r.words.p) {
+        r.words.alloc(RES_PART_WORDS + RES_TOT_WORDS);
+        r.epoch = 0xffffffffu;   // cleared below before the first use
+    }
+    if (!r.ctl.p) r.ctl.alloc(sizeof(ResColOut) * 64 + sizeof(double) * 64 + 8);
+    if (!r.h_ctl) TMI_HIP(hipHostMalloc((void **)&r.h_ctl, r.ctl.n));
+    double *d_om = (double *)(r.ctl.p + sizeof(ResColOut) * 64);
+    double *h_om = (double *)(r.h_ctl + sizeof(ResColOut) * 64);
+    a.out = (ResColOut *)r.ctl.p;
+    a.abort_flag = (int *)(d_om + 64);
+    a.pub_p = r.pub_p.p;
+    a.pub_s = r.pub_s.p;
+    a.rd0 = r.rd0.p;
+    a.x64 = r.x64.p;
+    a.part = r.words.p;
+    a.tot = r.words.p + RES_PART_WORDS;
+    const size_t lds = (((size_t)l.nu * plan.kc * sin + 15) & ~(size_t)15) + res_lds_fixed(plan.kc);
+    // reductions of one launch, at most: eight per iteration (replacements
+    // included) and those of the replacements between iterations
+    const unsigned need = (unsigned)std::min<long>(8l * cap + 8192, 0x7fffffffl);
+    int notconv = 0;
+    for (int q0 = 0; q0 < nq; q0 += plan.K) {
+        a.K = std::min(plan.K, nq - q0);
+        a.q0 = q0;
+        if (r.epoch > 0xffffffffu - need) {
+            TMI_HIP(hipMemsetAsync(r.words.p, 0, r.words.bytes(), st));
+            r.epoch = 0;
+        }
+        a.epoch = r.epoch;
+        r.epoch += need;
+        // omegas and the cleared abort word in one upload
+        for (int c = 0; c < 64; c++) h_om[c] = mf && c < a.K ? h_omega[q0 + c] : 0.0;
+        *(int *)(h_om + 64) = 0;
+        TMI_HIP(hipMemcpyAsync(d_om, h_om, sizeof(double) * 64 + 8, hipMemcpyHostToDevice, st));
+        a.omega = mf ? d_om : nullptr;
+        const bool ok = cg ? launch_resident_cg(vk, plan.cl, plan.E, bil, mf, a, lds, st)
+                           : launch_resident_bicg(vk, plan.cl, plan.E, a, lds, st);
+        if (!ok) return -1;
+        TMI_HIP(hipMemcpyAsync(r.h_ctl, r.ctl.p, r.ctl.n, hipMemcpyDeviceToHost, st));
+        TMI_HIP(hipStreamSynchronize(st));
+        e.n_sync++;
+        if (*(int *)(h_om + 64)) return -1;
+        const ResColOut *out = (const ResColOut *)r.h_ctl;
+        for (int c = 0; c < a.K; c++) {
+            const double b2 = out[c].bnorm2, r2 = out[c].res2;
+            const bool conv = b2 == 0.0 || r2 <= a.tol2 * b2;
+            if (!conv) notconv++;
+            stats[q0 + c].iters = out[c].iters;
+            stats[q0 + c].sweeps = out[c].sweeps;
+            stats[q0 + c].relres = b2 > 0.0 ? std::sqrt(r2 / b2) : 0.0;
+            stats[q0 + c].converged = conv ? 1 : 0;
+            e.last_iters += out[c].iters;
+        }
+    }
+    return notconv;
+}
+
+}  // namespace tmi

@@ -88,6 +88,15 @@ struct Solver {
         DBuf<int> cols;                // column maps of compaction (2 x 64)
         int *h_flags = nullptr;        // pinned host mirror of per-column ints (inner, outer)
         double *h_dbl = nullptr;       // pinned host mirror of per-column doubles
+        // resident solve (krylov_resident.hpp): published vectors, FP64
+        // solution, stamped words and their running stamp, per-column results
+        struct Resident {
+            DBuf<char> pub_p, pub_s, rd0, x64, ctl;
+            DBuf<unsigned long long> words;
+            unsigned epoch = 0;
+            char *h_ctl = nullptr;
+        } res;
+        int res_md = -1;               // mode of the last solve, if it ran resident
         GmresWork *gm = nullptr;       // GMRES workspace (allocated by the first GMRES solve)
         double last_solve_ms = 0.0, last_iters = 0.0;
         // instantiated graphs of the check period's launch sequence, keyed by
@@ -113,6 +122,10 @@ struct Solver {
     };
     Exec ex;                           // default context (library stream)
     std::mutex prep_mu;                // lazy preconditioner setup
+    // the caller chose details of the launch sequence (tile, row schedule,
+    // SpMM variant, compaction, graph replay), or the autotuner found it
+    // faster: solves then take it instead of the resident kernel
+    bool launch_sequence = false;
 
     ~Solver();
     VKind vk64() const { return cplx ? VK_C64 : VK_R64; }
@@ -165,6 +178,25 @@ struct Solver {
     Exec::Work &ensure_work(Exec &e, int K, int md, bool alt = false);
     int solve_tile(Exec &e, int K, int kc, tmi_colstat *stats, void *d_x, int ld, int q0, int md,
                    const double *h_omega);
+    struct ResPlan {
+        int K = 0;    // columns per launch (0: the launch sequence)
+        int nr = 1;   // ranks (workgroups) per team
+        int kc = 1;   // columns per team, a power of two
+        int cl = 1;   // columns per lane
+        int E = 1;    // rows per thread
+    };
+    ResPlan resident_plan(int nq, int md);
+    static size_t resident_fixed_bytes();   // words and results, whatever the block
+    int solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats,
+                       int md, const double *h_omega);
+    // operators in the slice order of a resident layout, per operator kind
+    // and number of ranks; valid until the next assembly
+    enum OpKind { OPK_32, OPK_64, OPK_P32, OPK_P64, OPK_MF32, OPK_MF64, OPK_N };
+    struct SliceOp {
+        DBuf<char> v;
+        bool valid = false;
+    } slice_op[OPK_N][9];
+    const void *sliced(OpKind k, const ResLayout &l, int nr);   // caller holds prep_mu
     // GMRES(20) in FP64 on tiles of the columns (gmres.hip); every mode
     int gmres_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats);
     int count_active(Exec &e, const int *d_flags, int K);
