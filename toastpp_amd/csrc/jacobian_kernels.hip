@@ -10,10 +10,11 @@
 // G_i = aphi on N(i) (nm x d).  One workgroup per node: it builds A_i, B_i
 // in LDS from the element integrals, then for each chunk of detectors
 // gathers G into LDS and forms H = G A, K = G B, and for each chunk of
-// sources gathers F and forms P for the linked pairs of the two chunks,
-// written node-major (one contiguous row of the intermediate per node).  A tiled transpose kernel
-// then scales by 1/proj (log data), negates and writes J in the reference
-// layout [dlnA/dmua | dlnA/dkappa ; dphase/dmua | dphase/dkappa].
+// sources gathers F and forms P for the linked pairs of the two chunks, scaled
+// by 1/proj (log data), negated and written to J in the reference layout
+// [dlnA/dmua | dlnA/dkappa ; dphase/dmua | dphase/dkappa].  This kernel takes
+// any neighbour count that fits the LDS of a CU; most meshes take
+// jacobian_tiles.hip instead (jacobian_tiles_pay).
 //
 // This file is compiled without floating-point contraction so that A_i and
 // B_i use the exact element integrals of the assembly; the GEMM loops opt in
@@ -21,8 +22,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdlib>
-#include <cstring>
 
 #include "fe_integrals.hpp"
 #include "jacobian.hpp"
@@ -37,18 +36,8 @@ constexpr int JAC_NT = 256;
 #endif
 constexpr int JAC_LDS_KIB = TMI_JAC_LDS_KIB;
 
-// J and the node-major intermediate are written once and read at most once:
-// streaming (nontemporal) accesses keep them out of the caches
-typedef double jac_dv2 __attribute__((ext_vector_type(2)));
+// J is written once: streaming (nontemporal) stores keep it out of the caches
 __device__ inline void st_stream(double *p, double v) { __builtin_nontemporal_store(v, p); }
-__device__ inline void st_stream(double2 *p, double2 v)
-{
-    __builtin_nontemporal_store(__builtin_bit_cast(jac_dv2, v), (jac_dv2 *)p);
-}
-__device__ inline double2 ld_stream(const double2 *p)
-{
-    return __builtin_bit_cast(double2, __builtin_nontemporal_load((const jac_dv2 *)p));
-}
 
 struct JacDims {
     int n, nq, nm, nqm, dmax, chunk, ldd, lda;
@@ -77,10 +66,9 @@ static size_t jac_lds_doubles(int dmax, int chunk)
     return (size_t)2 * dmax * dmax + jac_region_doubles(dmax, chunk) + (dmax + 1) / 2 + 1;
 }
 
-// Output of the direct variant: J (complex: 2nqm x 2n, [Re; Im] x [mua |
-// kappa]) or the CW pair Jmua / Jkap (nqm x n each, either may be absent),
-// scaled by 1/proj (log data) and negated, as k_jac_transpose /
-// k_jac_transpose_cw write them from the intermediate.
+// Output: J (complex: 2nqm x 2n, [Re; Im] x [mua | kappa]) or the CW pair
+// Jmua / Jkap (nqm x n each, either may be absent), scaled by 1/proj (log
+// data) and negated.
 struct JacOut {
     double *J, *Jkap;
     const double *proj;
@@ -124,7 +112,7 @@ __device__ inline int xcd_node(int b, int n)
     return x * q + min(x, r) + s;
 }
 
-template <int DIM, bool DIRECT>
+template <int DIM>
 __global__ void __launch_bounds__(JAC_NT) k_jac_nodes(JacDims jd, const int *__restrict__ rowptr,
                                                   const int *__restrict__ colidx, const int *__restrict__ n2e_ptr,
                                                   const int *__restrict__ n2e, const int *__restrict__ el,
@@ -132,13 +120,12 @@ __global__ void __launch_bounds__(JAC_NT) k_jac_nodes(JacDims jd, const int *__r
                                                   const double2 *__restrict__ dphi,   // [n][ldd]
                                                   const double2 *__restrict__ aphi,   // [n][lda]
                                                   const int *__restrict__ lk,         // [nq][nm] link or -1
-                                                  double2 *__restrict__ Pt,           // [n][nqm][2]
                                                   JacOut jo)
 {
     constexpr int NN = DIM + 1;
     constexpr int GS = DIM == 3 ? GEO3 : GEO2;
     extern __shared__ double lds[];
-    const int i = DIRECT ? xcd_node(blockIdx.x, jd.n) : blockIdx.x;
+    const int i = xcd_node(blockIdx.x, jd.n);
     const int tid = threadIdx.x;
     const int dmax = jd.dmax, nq = jd.nq, nm = jd.nm, C = jd.chunk;
     double *A = lds, *B = A + dmax * dmax;
@@ -189,7 +176,6 @@ __global__ void __launch_bounds__(JAC_NT) k_jac_nodes(JacDims jd, const int *__r
             __syncthreads();
         }
     }
-    double2 *out = Pt + (size_t)i * jd.nqm * 2;
     for (int m0 = 0; m0 < nm; m0 += C) {
         const int mc = min(C, nm - m0);
         // detector chunk G on the neighbour set
@@ -239,93 +225,10 @@ __global__ void __launch_bounds__(JAC_NT) k_jac_nodes(JacDims jd, const int *__r
                         pr += fv.x * kv.x - fv.y * kv.y;
                         pi += fv.x * kv.y + fv.y * kv.x;
                     }
-                    if constexpr (DIRECT) {
-                        jac_emit(jo, jd.n, jd.nqm, i, k, mr, mi, pr, pi);
-                    } else {
-                        st_stream(out + 2 * k, make_double2(mr, mi));
-                        st_stream(out + 2 * k + 1, make_double2(pr, pi));
-                    }
+                    jac_emit(jo, jd.n, jd.nqm, i, k, mr, mi, pr, pi);
                 }
             }
             __syncthreads();
-        }
-    }
-}
-
-// J[k][i] = -Re(P_mua/proj_k), J[k+nqm][i] = -Im(.), J[k][n+i] = -Re(P_kap/proj_k),
-// J[k+nqm][n+i] = -Im(.)  (DATA_LOG; without log the division is skipped).
-// Tiles of 64 nodes x 16 measurements through LDS: the reads take 512-byte
-// runs of one node's measurements, the writes 512-byte runs of one J row.
-constexpr int TJK = 16;
-__global__ void __launch_bounds__(256) k_jac_transpose(int n, int nqm, const double2 *__restrict__ Pt,
-                                                       const double2 *__restrict__ proj, int logscale,
-                                                       double *__restrict__ J)
-{
-    __shared__ double2 tm[64][TJK + 1], tk[64][TJK + 1];
-    const int i0 = blockIdx.x * 64, k0 = blockIdx.y * TJK;
-    const int t = threadIdx.x;
-    // read: node r, measurement c (2 values each)
-    for (int e = t; e < 64 * TJK; e += 256) {
-        const int r = e / TJK, c = e % TJK;
-        const int i = i0 + r, k = k0 + c;
-        if (i < n && k < nqm) {
-            tm[r][c] = ld_stream(Pt + ((size_t)i * nqm + k) * 2);
-            tk[r][c] = ld_stream(Pt + ((size_t)i * nqm + k) * 2 + 1);
-        }
-    }
-    __syncthreads();
-    const size_t ld = 2 * (size_t)n;
-    for (int e = t; e < 64 * TJK; e += 256) {
-        const int c = e / 64, r = e % 64;
-        const int k = k0 + c, i = i0 + r;
-        if (k < nqm && i < n) {
-            double2 a = tm[r][c], b = tk[r][c];
-            if (logscale) {
-                const double2 p = proj[k];
-                const double den = p.x * p.x + p.y * p.y;
-                a = make_double2((a.x * p.x + a.y * p.y) / den, (a.y * p.x - a.x * p.y) / den);
-                b = make_double2((b.x * p.x + b.y * p.y) / den, (b.y * p.x - b.x * p.y) / den);
-            }
-            st_stream(J + (size_t)k * ld + i, -a.x);
-            st_stream(J + (size_t)(k + nqm) * ld + i, -a.y);
-            st_stream(J + (size_t)k * ld + n + i, -b.x);
-            st_stream(J + (size_t)(k + nqm) * ld + n + i, -b.y);
-        }
-    }
-}
-
-// CW (GenerateJacobian_cw_mesh, jacobian.cc:727-790, then the log row scaling
-// of :160-186): from the intermediate of real fields, Jmua[k][i] =
-// -P_mua * (1/proj_k), Jkap[k][i] = -P_kap * (1/proj_k) (without log the
-// factor is dropped); either output may be absent.  Same tiling as above.
-__global__ void __launch_bounds__(256) k_jac_transpose_cw(int n, int nqm, const double2 *__restrict__ Pt,
-                                                          const double *__restrict__ proj, int logscale,
-                                                          double *__restrict__ Jmua, double *__restrict__ Jkap)
-{
-    __shared__ double tm[64][TJK + 1], tk[64][TJK + 1];
-    const int i0 = blockIdx.x * 64, k0 = blockIdx.y * TJK;
-    const int t = threadIdx.x;
-    for (int e = t; e < 64 * TJK; e += 256) {
-        const int r = e / TJK, c = e % TJK;
-        const int i = i0 + r, k = k0 + c;
-        if (i < n && k < nqm) {
-            tm[r][c] = ld_stream(Pt + ((size_t)i * nqm + k) * 2).x;
-            tk[r][c] = ld_stream(Pt + ((size_t)i * nqm + k) * 2 + 1).x;
-        }
-    }
-    __syncthreads();
-    for (int e = t; e < 64 * TJK; e += 256) {
-        const int c = e / 64, r = e % 64;
-        const int k = k0 + c, i = i0 + r;
-        if (k < nqm && i < n) {
-            double a = -tm[r][c], b = -tk[r][c];
-            if (logscale) {
-                const double ip = 1.0 / proj[k];
-                a *= ip;
-                b *= ip;
-            }
-            if (Jmua) st_stream(Jmua + (size_t)k * n + i, a);
-            if (Jkap) st_stream(Jkap + (size_t)k * n + i, b);
         }
     }
 }
@@ -466,21 +369,28 @@ void launch_real_to_cplx(long rows, int cols, const double *src, int ld, double 
     TMI_LAUNCH_CHECK();
 }
 
-// How the nodal Jacobian kernel's output reaches J (TMI_JAC_MODE, read
-// once): by default the node kernel writes J itself (nodes dealt to the XCDs
-// in contiguous runs, so that the 8-byte entries of neighbouring nodes fill
-// cache lines in one L2); "two" keeps the earlier layout, a node-major
-// intermediate of n nqm 32 B (streaming stores) and one tiled transpose.
-bool jacobian_two_pass()
+// The matrix-core kernel pads the neighbours to 16 or 32.  Up to 16 it was
+// faster at every size measured (ms, per-node kernel against it: 3,169 nodes
+// 2 x 2 links 0.030 / 0.027, 32 x 32 0.092 / 0.055; 59,319 nodes 0.517 / 0.170
+// and 1.788 / 0.952).  With longer rows most of the 32 may be padding: on
+// triangulated random points (mean 7, longest 17; 40,000 nodes) 0.187 / 0.396
+// at 4 x 4 links and 1.08 / 1.49 at 32 x 32, on tetrahedra (mean 16.3, longest
+// 32; 59,887 nodes) 0.735 / 0.659 and 3.61 / 2.57, but with 2,844 nodes 0.056 /
+// 0.060 at 8 x 8 links against 0.068 / 0.064 at 16 x 16.
+static bool jacobian_tiles_pay(const Mesh &m, int nq, int nm, int dmax)
 {
-    static const bool two = getenv("TMI_JAC_MODE") && !strcmp(getenv("TMI_JAC_MODE"), "two");
-    return two;
+    return dmax <= 16 || (dmax <= 32 && (long)m.nnz >= 12L * m.n && (long)nq * nm >= 256);
 }
 
-void launch_jacobian_nodal(const Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
-                           int nqm, const double *d_proj, int logscale, double *d_Pt, double *d_J, int dmax,
-                           hipStream_t st, bool cw, double *d_Jkap)
+void launch_jacobian_nodal(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
+                           int nqm, const double *d_proj, int logscale, double *d_J, int dmax, hipStream_t st, bool cw,
+                           double *d_Jkap)
 {
+    if (cw && !d_J && !d_Jkap) return;
+    if (jacobian_tiles_pay(m, nq, nm, dmax)) {
+        launch_jacobian_tiles(m, nq, nm, d_dphi, ldd, d_aphi, lda, nqm, d_proj, logscale, d_J, dmax, st, cw, d_Jkap);
+        return;
+    }
     // LDS row stride: the neighbour count rounded up to odd, so that the
     // rows of A, B, W, H read by consecutive lanes start in different banks
     dmax |= 1;
@@ -497,23 +407,12 @@ void launch_jacobian_nodal(const Mesh &m, int nq, int nm, const double *d_dphi, 
               "nodal Jacobian: %d neighbours per node exceed the LDS of one CU", dmax);
     const JacDims jd{m.n, nq, nm, nqm, dmax, chunk, ldd, lda};
     const JacOut jo{d_J, d_Jkap, d_proj, logscale, cw ? 1 : 0};
-    const bool two = jacobian_two_pass();
-#define JN(D, DIR)                                                                                                  \
-    hipLaunchKernelGGL((k_jac_nodes<D, DIR>), dim3(m.n), dim3(JAC_NT), lds, st, jd, m.rowptr.p, m.colidx.p,          \
-                       m.n2e_ptr.p, m.n2e.p, m.elist.p, m.geo.p, (const double2 *)d_dphi, (const double2 *)d_aphi,     \
-                       m.d_lk.p, (double2 *)d_Pt, jo);
-    if (m.dim == 3) { if (two) JN(3, false) else JN(3, true) }
-    else { if (two) JN(2, false) else JN(2, true) }
+#define JN(D)                                                                                                       \
+    hipLaunchKernelGGL((k_jac_nodes<D>), dim3(m.n), dim3(JAC_NT), lds, st, jd, m.rowptr.p, m.colidx.p, m.n2e_ptr.p,  \
+                       m.n2e.p, m.elist.p, m.geo.p, (const double2 *)d_dphi, (const double2 *)d_aphi, m.d_lk.p, jo);
+    if (m.dim == 3) JN(3)
+    else JN(2)
 #undef JN
-    TMI_LAUNCH_CHECK();
-    if (!two) return;
-    dim3 g((m.n + 63) / 64, (nqm + TJK - 1) / TJK);
-    if (cw)
-        hipLaunchKernelGGL(k_jac_transpose_cw, g, dim3(256), 0, st, m.n, nqm, (const double2 *)d_Pt, d_proj, logscale,
-                           d_J, d_Jkap);
-    else
-        hipLaunchKernelGGL(k_jac_transpose, g, dim3(256), 0, st, m.n, nqm, (const double2 *)d_Pt,
-                           (const double2 *)d_proj, logscale, d_J);
     TMI_LAUNCH_CHECK();
 }
 

@@ -55,11 +55,14 @@ struct Mesh {
     std::vector<int> h_bnd;
     QM qm;
     // device copy of the QM link list for the Jacobian (row pointer, source
-    // and detector per link; rebuilt when the QM changes) and the Jacobian's
-    // node-major intermediate, kept between calls
+    // and detector per link; rebuilt when the QM changes)
     bool links_valid = false;
     DBuf<int> d_lptr, d_lq, d_lm, d_lk;   // link list; d_lk[q * nm + m] = link of (q, m) or -1
-    DBuf<double> jac_ws;
+    // nodal Jacobian: the nodes' element-integral matrices as operands of the
+    // matrix cores (jacobian_tiles.hip), built on its first call
+    DBuf<double> jac_ops;
+    bool jac_ops_ok = false;
+    std::mutex jac_mu;
     // node orders of the solvers' private copies of the system (order.cpp),
     // one per kind (ORDER_NATURAL, ORDER_MORTON, ORDER_CLUSTER): row r of the relabelled
     // system is node perm[r]; its CSR pattern with slot[k] = nonzero of the
