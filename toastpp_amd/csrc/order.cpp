@@ -13,6 +13,8 @@
 #include <iterator>
 #include <cstdint>
 #include <numeric>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "krylov.hpp"
@@ -254,6 +256,17 @@ static void split_ranks(int dim, int n, int nr, int lo, int hi, const double *x,
             const double u = x[(size_t)node[p] * dim + d], v = x[(size_t)node[q] * dim + d];
             return u != v ? u < v : p < q;
         });
+    if (hi - lo >= nr / 4 && b - a >= 4096) {   // the halves are independent: up to eight threads
+        std::thread half;
+        try {
+            half = std::thread([&] { split_ranks(dim, n, nr, lo, mid, x, node, row); });
+        } catch (const std::system_error &) {   // none to be had
+        }
+        split_ranks(dim, n, nr, mid, hi, x, node, row);
+        if (half.joinable()) half.join();
+        else split_ranks(dim, n, nr, lo, mid, x, node, row);
+        return;
+    }
     split_ranks(dim, n, nr, lo, mid, x, node, row);
     split_ranks(dim, n, nr, mid, hi, x, node, row);
 }
