@@ -30,8 +30,8 @@ struct Raster {
     DBuf<int> gi_rp, gi_ci;            // GI (glen x blen CSR), built on first use
     DBuf<double> gi_val;
     bool gi_built = false;
-    DBuf<double> fgv;                  // Jacobian scratch: fields on the grid
-    DBuf<double> fgs;                  // Jacobian scratch: fields + gradients on the grid voxels inside the mesh
+    DBuf<double> fgv;                  // Jacobian and gradient scratch: fields on the grid, column by column
+    DBuf<double> fgs;                  // gradient through G: values + gradients at the grid points inside the mesh
     DBuf<int> ncols;                   // nlen x 2^dim: grid points of NodeMapMatrix (-1 unused)
     DBuf<double> nw;                   // nlen x 2^dim: their interpolation weights
     int ncols_nodemap = 0;             // 2^dim once built
