@@ -4,7 +4,7 @@
 //
 // A launch sequence pays, per iteration, five dependent kernels (25-30 us at
 // a few thousand to 30k nodes, where the data of an iteration moves in 2-5
-// us), and streams every Krylov vector through memory.  Here one 1024-thread
+// us), and streams every Krylov vector through memory.  Here one 512-thread
 // workgroup per CU owns a fixed set of rows for the whole solve: x, r and the
 // SpMM result of its elements stay in registers, the direction p in LDS;
 // only the vector the next SpMM gathers is published to memory, and the
@@ -12,7 +12,7 @@
 //
 // Teams: the workgroups form T teams of nr = 256/T ranks; team t owns kc
 // consecutive columns, rank r of a team a contiguous range of rows (ResLayout,
-// built on the host once per mesh order and nr).  Workgroup b runs on XCD
+// built on the GPU once per mesh order and nr).  Workgroup b runs on XCD
 // b % 8 and takes the logical id (b % 8) 32 + b / 8, so a team of up to 32
 // ranks shares one XCD and a wider one whole XCDs.  Teams never exchange
 // anything: each runs until its own columns are done.

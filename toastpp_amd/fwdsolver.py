@@ -73,6 +73,9 @@ class FwdSolver:
         L.call("tmi_solver_set_mode", self._h, int(m))
 
     def SetTile(self, tile):
+        """columns per tile of the launch sequence (0: by the column count);
+        another value than 0 also keeps small blocks off the resident kernel,
+        as SetRowsPerWave, SetSpmmVariant, SetCompaction and SetGraphs do"""
         L.call("tmi_solver_set_tile", self._h, int(tile))
 
     def SetOrder(self, order):
