@@ -15,8 +15,9 @@ namespace tmi {
 void launch_jacobian_nodal(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
                            int nqm, const double *d_proj, int logscale, double *d_J, int dmax, hipStream_t st,
                            bool cw = false, double *d_Jkap = nullptr);
-// the same for dmax <= 32, on the matrix cores (cw: at least one block)
-void launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
+// the same for dmax <= 32, on the matrix cores (cw: at least one block); false
+// if there is no memory for its operands, with nothing launched
+bool launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
                            int nqm, const double *d_proj, int logscale, double *d_J, int dmax, hipStream_t st, bool cw,
                            double *d_Jkap);
 // Element-basis Jacobian: d_J (2 nqm) x (2 elen) row-major, or with cw the

@@ -387,10 +387,9 @@ void launch_jacobian_nodal(Mesh &m, int nq, int nm, const double *d_dphi, int ld
                            double *d_Jkap)
 {
     if (cw && !d_J && !d_Jkap) return;
-    if (jacobian_tiles_pay(m, nq, nm, dmax)) {
-        launch_jacobian_tiles(m, nq, nm, d_dphi, ldd, d_aphi, lda, nqm, d_proj, logscale, d_J, dmax, st, cw, d_Jkap);
+    if (jacobian_tiles_pay(m, nq, nm, dmax) &&
+        launch_jacobian_tiles(m, nq, nm, d_dphi, ldd, d_aphi, lda, nqm, d_proj, logscale, d_J, dmax, st, cw, d_Jkap))
         return;
-    }
     // LDS row stride: the neighbour count rounded up to odd, so that the
     // rows of A, B, W, H read by consecutive lanes start in different banks
     dmax |= 1;

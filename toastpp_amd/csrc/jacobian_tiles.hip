@@ -334,7 +334,7 @@ __global__ void __launch_bounds__(JT_NT, 3) k_jac_tiles(JtArgs A)
     }
 }
 
-void launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
+bool launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
                            int nqm, const double *d_proj, int logscale, double *d_J, int dmax, hipStream_t st, bool cw,
                            double *d_Jkap)
 {
@@ -355,7 +355,16 @@ void launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ld
     const int part = (int)std::min<size_t>(m.n, JT_OPS_BYTES / per);
     const bool whole = part == m.n;
     std::unique_lock<std::mutex> lock(m.jac_mu);
-    if (m.jac_ops.n * sizeof(double) < part * per) m.jac_ops.alloc(part * per / sizeof(double));
+    if (m.jac_ops.n * sizeof(double) < part * per) {
+        try {
+            m.jac_ops.alloc(part * per / sizeof(double));
+        } catch (const Error &err) {
+            if (err.code != TMI_ERR_OOM) throw;
+            (void)hipGetLastError();
+            m.jac_ops.release();
+            return false;   // the per-node kernel needs none
+        }
+    }
     const size_t lds = (size_t)256 * (cw ? 1 : 2) * 2 * JT_LINE * sizeof(double);
     const long units = (long)a.tq * a.tm * a.nkind;
     for (int lo = 0; lo < m.n; lo += part) {
@@ -398,6 +407,7 @@ void launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ld
     }
     // the parts' operands are shared: the next call's stream may be another
     if (!whole) TMI_HIP(hipStreamSynchronize(st));
+    return true;
 }
 
 }  // namespace tmi
