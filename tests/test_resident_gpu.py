@@ -118,3 +118,31 @@ def test_resident_zero_column_and_cap(setups):
             assert a[0] == b[0] == 16 and not a[3]
             assert abs(a[2] - b[2]) <= 1e-13   # rounding of b - A x, relative to ||b||
         assert _compare(X, Xs) <= 1e-9   # the same iterates up to the order of the sums
+
+
+def test_resident_bicgstab_idle_columns(setups):
+    """A column that has met its recursive test waits for the next residual
+    replacement and may run on after it.  What the other columns of its team
+    do meanwhile must not matter: beside columns that need twice its
+    iterations it takes the same iterates, bit for bit, as beside others that
+    stop when it does (sources in a strongly absorbing half of the mesh, which
+    meet the FP32 test after about 20 iterations and fail the FP64 one)."""
+    mesh, _, _ = setups("ell9k")
+    nodes, _ = G.ellipsoid(80.0, 65.0, 90.0, 20)
+    mua, mus, ref = G.params(nodes, 7)
+    x = nodes[:, 0]
+    sol = T.Solution(np.where(x > 0, 1e4 * mua, mua), mus, ref)
+    fast, slow = np.where(x > 24.0)[0], np.where(x < -24.0)[0]
+
+    def rhs(centres):
+        d2 = ((nodes[:, None, :] - nodes[None, centres, :]) ** 2).sum(2)
+        return np.ascontiguousarray(np.exp(-d2 / 8.0).astype(complex))
+    f = rhs(fast[np.arange(64) * len(fast) // 64])
+    mixed = rhs(slow[np.arange(64) * len(slow) // 64])
+    mixed[:, ::2] = f[:, ::2]
+    Xf, stf, _ = _solve(mesh, sol, f, "BICGSTAB", "mixed", "DIAG", False)
+    Xm, stm, counts = _solve(mesh, sol, mixed, "BICGSTAB", "mixed", "DIAG", False)
+    assert counts[0] <= 6 and counts[1] == 0   # resident
+    assert max(s[0] for s in stf) + 8 < max(s[0] for s in stm[1::2])
+    assert [s[0] for s in stf[::2]] == [s[0] for s in stm[::2]]
+    assert np.array_equal(Xf[:, ::2], Xm[:, ::2])

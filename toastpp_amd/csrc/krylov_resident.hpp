@@ -695,11 +695,16 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
                         p = first[j] ? r[e][j]
                                      : vadd(r[e][j], res_scale(vsub(pv[e][j], res_scale(y[e][j], om[j])), br[j]));
                     }
-                    if (act[j]) {
-                        if constexpr (M == RES_BICG) pv[e][j] = p;
+                    if constexpr (M == RES_BICG) {
+                        // the stage holds s of the last iteration: an idle
+                        // column's p goes back too, for its product below
+                        if (act[j]) pv[e][j] = p;
+                        else p = pv[e][j];
                         sp[j] = p;
-                        if (a.nr > 1) st_pub(pp + j, p);
+                    } else if (act[j]) {
+                        sp[j] = p;
                     }
+                    if (act[j] && a.nr > 1) st_pub(pp + j, p);
                 }
             }
         }
@@ -708,7 +713,9 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
         if (a.nr > 1) load_halo(Pt);
         // ---- y = A p and its product
         FRESH;
-        // (an inactive column's p is unchanged, so its product is too)
+        // (an idle column's p is unchanged, here and where it is published, so
+        // its product is too: BiCGSTAB needs it if the column runs on after a
+        // residual replacement)
         CLEAR_D;
         products(y);
         FOR_E if (ON(e)) {
