@@ -83,6 +83,9 @@ const char *tmi_last_error(void);
 int tmi_device_info(char *name, int name_len, double *hbm_gib);
 /* Wait for all queued GPU work of the library. */
 int tmi_synchronize(void);
+/* For tests of the out-of-memory paths: the library's own device allocations
+ * of the calling thread above `bytes` fail with TMI_ERR_OOM (0: no limit). */
+int tmi_test_alloc_limit(double bytes);
 /* Device buffers for the *_device entry points (no reference counterpart;
  * plumbing for callers without their own allocator). */
 int tmi_device_alloc(unsigned long long bytes, void **ptr);

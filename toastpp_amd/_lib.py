@@ -58,6 +58,7 @@ DP = C.POINTER(C.c_double)
 _SIGS = {
     "tmi_device_info": [C.c_char_p, C.c_int, DP],
     "tmi_synchronize": [],
+    "tmi_test_alloc_limit": [C.c_double],
     "tmi_device_alloc": [C.c_ulonglong, PP],
     "tmi_device_free": [P],
     "tmi_memcpy_h2d": [P, P, C.c_ulonglong],

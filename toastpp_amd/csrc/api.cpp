@@ -14,6 +14,7 @@ namespace tmi {
 
 static thread_local std::string g_last_error;
 thread_local long long g_launch_calls = 0;
+thread_local size_t g_alloc_limit = (size_t)-1;
 void set_last_error(const std::string &msg) { g_last_error = msg; }
 
 Context &Context::get()
@@ -101,6 +102,13 @@ int tmi_synchronize(void)
 {
     API_BEGIN
     TMI_HIP(hipStreamSynchronize(Context::get().stream));
+    API_END
+}
+
+int tmi_test_alloc_limit(double bytes)
+{
+    API_BEGIN
+    g_alloc_limit = bytes > 0 ? (size_t)bytes : (size_t)-1;
     API_END
 }
 

@@ -64,7 +64,10 @@ extern thread_local long long g_launch_calls;
 
 void set_last_error(const std::string &msg);
 
-// Owning device allocation.
+// largest device allocation of this thread (tests of the out-of-memory paths)
+extern thread_local size_t g_alloc_limit;
+
+// Owning device allocation; one that failed leaves it empty.
 template <class T>
 struct DBuf {
     T *p = nullptr;
@@ -84,8 +87,18 @@ struct DBuf {
     {
         if (count == n && p) return;
         release();
+        if (!count) return;
+        if (count > g_alloc_limit / sizeof(T))
+            fail(TMI_ERR_OOM, "allocation of %zu bytes above the limit of %zu", count * sizeof(T), g_alloc_limit);
+        void *q = nullptr;
+        const hipError_t e = hipMalloc(&q, count * sizeof(T));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();   // reported here, not by the next launch
+            fail(e == hipErrorOutOfMemory ? TMI_ERR_OOM : TMI_ERR_DEVICE, "device allocation of %zu bytes failed: %s",
+                 count * sizeof(T), hipGetErrorString(e));
+        }
+        p = (T *)q;
         n = count;
-        if (count) TMI_HIP(hipMalloc((void **)&p, count * sizeof(T)));
     }
     void release()
     {

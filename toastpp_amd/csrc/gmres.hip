@@ -366,19 +366,21 @@ struct GmresWork {
     void ensure(int n_, int K_, size_t es_)
     {
         if (K == K_ && n == n_ && es == es_) return;
-        K = K_, n = n_, es = es_;
-        G = (int)std::min<size_t>(GM_MAXG, std::max<size_t>(1, ((size_t)n * K + 4 * GM_BLOCK - 1) / (4 * GM_BLOCK)));
-        const size_t nk = (size_t)n * K;
+        K = 0;   // until all of it is there
+        n = n_, es = es_;
+        G = (int)std::min<size_t>(GM_MAXG, std::max<size_t>(1, ((size_t)n * K_ + 4 * GM_BLOCK - 1) / (4 * GM_BLOCK)));
+        const size_t nk = (size_t)n * K_;
         V.alloc(nk * (GM_RESTART + 1) * es);
         mb.alloc(nk * es);
-        H.alloc((size_t)K * GM_RESTART * (GM_RESTART + 1) * es);
-        s.alloc((size_t)K * (GM_RESTART + 1) * es);
-        c1.alloc((size_t)K * GM_RESTART * es);
-        c2.alloc((size_t)K * GM_RESTART * es);
-        y.alloc((size_t)K * GM_RESTART * es);
-        part.alloc((size_t)G * 2 * K * es);
-        dsc.alloc((size_t)D_NSLOT * K);
-        isc.alloc((size_t)G_NSLOT * K);
+        H.alloc((size_t)K_ * GM_RESTART * (GM_RESTART + 1) * es);
+        s.alloc((size_t)K_ * (GM_RESTART + 1) * es);
+        c1.alloc((size_t)K_ * GM_RESTART * es);
+        c2.alloc((size_t)K_ * GM_RESTART * es);
+        y.alloc((size_t)K_ * GM_RESTART * es);
+        part.alloc((size_t)G * 2 * K_ * es);
+        dsc.alloc((size_t)D_NSLOT * K_);
+        isc.alloc((size_t)G_NSLOT * K_);
+        K = K_;
     }
 };
 

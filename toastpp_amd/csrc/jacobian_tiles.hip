@@ -360,8 +360,6 @@ bool launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ld
             m.jac_ops.alloc(part * per / sizeof(double));
         } catch (const Error &err) {
             if (err.code != TMI_ERR_OOM) throw;
-            (void)hipGetLastError();
-            m.jac_ops.release();
             return false;   // the per-node kernel needs none
         }
     }

@@ -246,9 +246,7 @@ Solver::Exec::Work &Solver::ensure_work(Exec &e, int K, int md, bool alt)
     if (!e.h_dbl) TMI_HIP(hipHostMalloc((void **)&e.h_dbl, sizeof(double) * S_NSLOT * 64));
     if (!e.cols.p) e.cols.alloc(128);
     if (w.K == K && w.n == n && w.vk_in == vin) return w;
-    w.K = K;
-    w.n = n;
-    w.vk_in = vin;
+    w.K = 0;   // until all of it is there
     // reduction workgroups: a multiple of 8 (one slice per XCD), enough to
     // fill the GPU, few enough that the per-block partials stay small.  The
     // narrow tiles' SpMMs walk rows (a chain of dependent row-pointer,
@@ -267,6 +265,9 @@ Solver::Exec::Work &Solver::ensure_work(Exec &e, int K, int md, bool alt)
     if (K == 64 && vin == VK_C32) w.rdq.alloc((size_t)n * 32);
     w.sc.alloc((size_t)S_NSLOT * K); w.osc.alloc((size_t)S_NSLOT * K);
     w.ic.alloc((size_t)I_NSLOT * K); w.oic.alloc((size_t)I_NSLOT * K);
+    w.K = K;
+    w.n = n;
+    w.vk_in = vin;
     return w;
 }
 
