@@ -12,8 +12,8 @@
 #include <array>
 #include <iterator>
 #include <cstdint>
+#include <exception>
 #include <numeric>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -232,9 +232,8 @@ static void row_block_unions(int n, const std::vector<int> &rp, const std::vecto
 // .. n hi / nr) at the ranks' middle, across the longest side of their
 // nodes' bounding box: compact parts with short boundaries.  The bounds of
 // fewer ranks are bounds of more, so one split into 256 serves every count.
-// (A range of the
-// clustered order would not do: its last rows are the ones no cluster took,
-// from all over the mesh.)
+// (A range of the clustered order would not do: its last rows are the ones no
+// cluster took, from all over the mesh.)
 static void split_ranks(int dim, int n, int nr, int lo, int hi, const double *x, const std::vector<int> &node,
                         std::vector<int> &row)
 {
@@ -260,7 +259,7 @@ static void split_ranks(int dim, int n, int nr, int lo, int hi, const double *x,
         std::thread half;
         try {
             half = std::thread([&] { split_ranks(dim, n, nr, lo, mid, x, node, row); });
-        } catch (const std::system_error &) {   // none to be had
+        } catch (const std::exception &) {   // no thread, or no memory for one: both halves here
         }
         split_ranks(dim, n, nr, mid, hi, x, node, row);
         if (half.joinable()) half.join();
