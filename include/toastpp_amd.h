@@ -172,9 +172,11 @@ int tmi_solver_set_mode(tmi_solver s, int mode);                /* TMI_MODE_* */
  * most) are solved by one cooperative kernel that keeps the Krylov vectors in
  * registers and LDS (no reference counterpart); larger ones by a launch
  * sequence on column tiles.  Naming a detail of the launch sequence -- tile,
- * rows per wave, SpMM variant, compaction, graphs -- selects it for every
- * solve of the handle; the autotuner keeps whichever is faster.  Same method,
- * recurrences and stopping tests; sums in another order.
+ * rows per wave, SpMM variant, compaction, graphs, its default value too --
+ * selects it for every solve of the handle; a tile of 0 (auto) takes the
+ * choice of a tile back, and no other.  The autotuner keeps whichever is
+ * faster for its mode and number of columns (until the next set_linsolver).
+ * Same method, recurrences and stopping tests; sums in another order.
  * Column tile of the launch sequence (RHS columns per Krylov block; 0 = auto) */
 int tmi_solver_set_tile(tmi_solver s, int tile);
 /* Node order of the solver's private copy of the system (no reference

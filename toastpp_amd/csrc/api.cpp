@@ -473,6 +473,7 @@ int tmi_solver_set_linsolver(tmi_solver h, const char *name, double tol)
     API_BEGIN
     Solver &s = S(h);
     NEED(name);
+    for (unsigned long long &t : s.tuned_sequence) t = 0;   // found with the other method
     if (!strcasecmp(name, "DIRECT")) {
         s.lsolver = s.cplx ? TMI_LSOLVER_BICGSTAB : TMI_LSOLVER_CG;
         s.tol = 1e-14;
@@ -529,7 +530,7 @@ int tmi_solver_set_tile(tmi_solver h, int tile)
     TMI_CHECK(tile == 0 || tile == 1 || tile == 2 || tile == 4 || tile == 8 || tile == 16 || tile == 32 || tile == 64,
               TMI_ERR_INVALID_ARG, "tile must be 0 (auto) or a power of two <= 64");
     S(h).tile = tile;
-    S(h).launch_sequence = tile != 0;
+    S(h).named = tile ? S(h).named | Solver::NAMED_TILE : S(h).named & ~Solver::NAMED_TILE;
     API_END
 }
 
@@ -575,7 +576,7 @@ int tmi_solver_set_rows_per_wave(tmi_solver h, int rows)
     API_BEGIN
     TMI_CHECK(rows >= 0 && rows <= 63, TMI_ERR_INVALID_ARG, "rows per wave must be 0 .. 63");
     S(h).rpw = rows;
-    S(h).launch_sequence = true;
+    S(h).named |= Solver::NAMED_ROWS;
     API_END
 }
 
@@ -587,7 +588,7 @@ int tmi_solver_set_spmm_variant(tmi_solver h, int variant)
               "(row blocks with shared gathers), 4 (row blocks, software-pipelined) or 5 (row blocks on the "
               "matrix cores)");
     S(h).spmm_variant = variant;
-    S(h).launch_sequence = true;
+    S(h).named |= Solver::NAMED_SPMM;
     API_END
 }
 
@@ -607,7 +608,7 @@ int tmi_solver_set_compaction(tmi_solver h, int min_width)
                   min_width == 16 || min_width == 32,
               TMI_ERR_INVALID_ARG, "compaction width must be 0 (off) or a power of two <= 32");
     S(h).compact_min = min_width;
-    S(h).launch_sequence = true;
+    S(h).named |= Solver::NAMED_COMPACTION;
     API_END
 }
 
@@ -900,7 +901,7 @@ int tmi_solver_set_graphs(tmi_solver h, int enable)
     API_BEGIN
     Solver &s = S(h);
     s.use_graphs = enable != 0;
-    s.launch_sequence = true;
+    s.named |= Solver::NAMED_GRAPHS;
     if (!s.use_graphs) s.ex.drop_graphs();
     API_END
 }

@@ -34,7 +34,8 @@ Solver::ResPlan Solver::resident_plan(int nq, int md)
     const VKind vk = mixed ? vk32() : vk64();
     const size_t sz = vbytes(vk);
     const bool wide = vk == VK_C64;
-    if (launch_sequence || lsolver == TMI_LSOLVER_GMRES || nq < 1 || nq > 64) return none;
+    if (named || tuning || lsolver == TMI_LSOLVER_GMRES || nq < 1 || nq > 64) return none;
+    if (tuned_sequence[md] >> (nq - 1) & 1) return none;
     if ((size_t)mesh->n * nq * sz > RES_MAX_BYTES) return none;
     int pow = 1;
     while (pow < nq) pow *= 2;

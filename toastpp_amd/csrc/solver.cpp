@@ -862,11 +862,11 @@ void Solver::autotune(int nq, const void *d_b, void *d_x, int ld, int *tile_out,
     // tile, row schedule and variant are those of the launch sequence; a
     // resident solve of the same right-hand sides is timed against the result
     struct Sequence {
-        bool &flag, was;
-        explicit Sequence(bool &f) : flag(f), was(f) { flag = true; }
-        ~Sequence() { flag = was; }
+        bool &flag;
+        explicit Sequence(bool &f) : flag(f) { flag = true; }
+        ~Sequence() { flag = false; }
     };
-    std::unique_ptr<Sequence> seq(new Sequence(launch_sequence));
+    std::unique_ptr<Sequence> seq(new Sequence(tuning));
     const size_t es = vbytes(vk64());
     auto zero_x = [&]() { TMI_HIP(hipMemset2DAsync(d_x, (size_t)ld * es, 0, (size_t)nq * es, mesh->n, st)); };
     // 1. row schedule and SpMM variant of the 64-column kernel (mixed mode;
@@ -947,12 +947,14 @@ void Solver::autotune(int nq, const void *d_b, void *d_x, int ld, int *tile_out,
         }
         tile = pick;
         seq.reset();
+        const unsigned long long bit = nq <= 64 ? 1ull << (nq - 1) : 0;
+        tuned_sequence[mode] &= ~bit;
         if (resident_plan(nq, mode).K > 0) {
             zero_x();
             solve(nq, d_b, d_x, ld, nullptr);   // its first run builds the layout
             zero_x();
             solve(nq, d_b, d_x, ld, nullptr);
-            launch_sequence = ex.last_solve_ms > best;
+            if (ex.last_solve_ms > best) tuned_sequence[mode] |= bit;
             best = std::min(best, ex.last_solve_ms);
         }
         if (ms_out) *ms_out = best;

@@ -122,10 +122,13 @@ struct Solver {
     };
     Exec ex;                           // default context (library stream)
     std::mutex prep_mu;                // lazy preconditioner setup
-    // the caller chose details of the launch sequence (tile, row schedule,
-    // SpMM variant, compaction, graph replay), or the autotuner found it
-    // faster: solves then take it instead of the resident kernel
-    bool launch_sequence = false;
+    // details of the launch sequence the caller has named, one bit each:
+    // solves then take it instead of the resident kernel
+    enum Named { NAMED_TILE = 1, NAMED_ROWS = 2, NAMED_SPMM = 4, NAMED_COMPACTION = 8, NAMED_GRAPHS = 16 };
+    unsigned named = 0;
+    // ... as do those the autotuner found it faster for: per mode, bit nq - 1
+    unsigned long long tuned_sequence[3] = {0, 0, 0};
+    bool tuning = false;   // the autotuner is timing the launch sequence
 
     ~Solver();
     VKind vk64() const { return cplx ? VK_C64 : VK_R64; }

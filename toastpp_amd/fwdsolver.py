@@ -75,7 +75,8 @@ class FwdSolver:
     def SetTile(self, tile):
         """columns per tile of the launch sequence (0: by the column count);
         another value than 0 also keeps small blocks off the resident kernel,
-        as SetRowsPerWave, SetSpmmVariant, SetCompaction and SetGraphs do"""
+        as any call of SetRowsPerWave, SetSpmmVariant, SetCompaction and
+        SetGraphs does for good; 0 takes back only the choice of a tile"""
         L.call("tmi_solver_set_tile", self._h, int(tile))
 
     def SetOrder(self, order):
