@@ -43,9 +43,11 @@
 // has read the earlier ones.
 //
 // Every wait is bounded (RES_TIMEOUT ticks of the 100 MHz counter and a
-// shared abort word): a rank that gives up sets the abort word, all others
-// see it in their polls, and the kernel ends without having written a field;
-// the host then runs the launch sequence.
+// shared abort word): a rank that gives up sets the abort word, the others
+// see it in their polls, and the kernel ends.  Columns of teams that had
+// finished are then written, rows of the others hold their initial guesses
+// (or, where only some ranks saw the abort at the very end, solutions): a
+// start for the launch sequence, which the host then runs.
 //
 // The arithmetic per element and the per-column recurrences (fin_column) are
 // the launch sequence's; sums over rows are grouped by thread, wave, rank in
@@ -84,7 +86,7 @@ struct ResColOut {
 };
 
 struct ResArgs {
-    int n, K, kc, nr;                // rows, columns of this launch, columns per team, ranks per team
+    int n, K, kc, nr;                // rows, columns, columns per team, ranks per team
     int maxit, ru;                   // iteration cap; inner iterations between residual replacements
     int mixed;
     int nu;                          // rows of the LDS stage (longest own + halo of a rank)
@@ -99,10 +101,9 @@ struct ResArgs {
     const double *op64;              // operator of the FP64 residual in slice order
     const void *idiag;               // inverse diagonal, or null; multi-frequency: the diagonal at omega = 1
     const double *omega;             // per column, or null
-    const void *b;                   // caller's right-hand sides [n][ld] (columns q0 ..)
+    const void *b;                   // caller's right-hand sides [n][ld]
     void *x;                         // caller's fields: initial guess in, solution out
     long ld;
-    int q0;
     void *pub_p, *pub_s;             // published vectors [T][n][kc]
     void *x64;                       // FP64 solution [T][n][kc], published
     void *rd0;                       // shadow residual of the FP64 BiCGSTAB [T][n][kc], private to its owner
@@ -544,7 +545,7 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
     // ---- right-hand side norms, initial guess published
     CLEAR_D;
     FOR_E if (ON(e)) {
-        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + a.q0 + c0 + c;
+        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + c0 + c;
         FOR_J if (c + j < ncol) {
             const V64 b = ((const V64 *)a.b)[node + j];
             d[0][j] += dotR(b, b);
@@ -587,7 +588,7 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
             bool any = false;
             FOR_J any |= OUT(I_ACTIVE, j) != 0;
             if (any) FOR_E if (ON(e)) {
-                const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + a.q0 + c0 + c;
+                const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + c0 + c;
                 V64 s[CL];
                 S64 w[CL];
                 FOR_J { s[j] = vzero<V64>(); w[j] = MF ? (S64)omg[min(c + j, ncol - 1)] : (S64)1; }
@@ -828,7 +829,7 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
     __syncthreads();
     FRESH;
     FOR_E if (ON(e)) {
-        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + a.q0 + c0 + c;
+        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + c0 + c;
         FOR_J if (c + j < ncol)((V64 *)a.x)[node + j] = ld_pub((const V64 *)X + AT(e) + j);
     }
     if (rank == 0 && tid < ncol) {

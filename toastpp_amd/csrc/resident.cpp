@@ -1,5 +1,5 @@
 // Host side of the resident solve (krylov_resident.hpp): when it is taken,
-// how the columns are split over launches and teams, and the launch itself.
+// how the columns are split over teams, and the launch itself.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -10,13 +10,12 @@
 namespace tmi {
 
 // When and how a solve runs resident.  Against the launch sequence (us per
-// iteration, 1 launch each; COCG/PCG/BiCGSTAB on disks and cylinders):
+// iteration; COCG/PCG/BiCGSTAB on disks and cylinders):
 //   n 3,169 real x 16: 7.5 / 31       n 31,525 c64 x 2 (BiCGSTAB): 24 / 97
 //   n 19,441 c32 x 24: 26 / 38        n 31,525 c64 x 16: 27 / 59
 //   n 31,525 c32 x 8: 24 / 39         n 103,267 c32 x 8: 42 / 54
 //   n 31,525 c32 x 32 (BiCGSTAB): 74 / 76    n 31,525 c32 x 64: 73 / 72
-//   n 50,653 c32 x 64 (2 launches): 126 / 95
-// so it is taken for blocks of up to RES_MAX_BYTES, in one launch.
+// so it is taken for blocks of up to RES_MAX_BYTES.
 static constexpr size_t RES_MAX_BYTES = 8500000;
 // Teams: one column per team keeps the reductions small and the ranks few
 // (n 19,441 x 24: 8 ranks 26 us, 32 ranks 28; n 31,525 c64 x 16: 16 ranks 27,
@@ -58,7 +57,6 @@ Solver::ResPlan Solver::resident_plan(int nq, int md)
         if (!l || l->nu == INT_MAX) continue;
         if ((((size_t)l->nu * kc * sz + 15) & ~(size_t)15) + res_lds_fixed(kc) > RES_LDS) continue;
         ResPlan p;
-        p.K = nq;
         p.nr = nr;
         p.kc = kc;
         p.cl = cl;
@@ -91,10 +89,10 @@ const void *Solver::sliced(OpKind k, const ResLayout &l, int nr)
     return o.v.p;
 }
 
-// Columns 0 .. nq-1 in cooperative launches of plan.K columns.  Returns the
-// number of columns above the tolerance, or -1 when a launch was refused or
-// gave up (the fields then hold initial guesses or finished columns, a valid
-// start for the launch sequence).
+// Columns 0 .. nq-1 in one cooperative launch.  Returns the number of columns
+// above the tolerance, or -1 when the launch was refused or gave up (the
+// fields then hold initial guesses or solutions, a valid start for the launch
+// sequence).
 int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld,
                            tmi_colstat *stats, int md, const double *h_omega)
 {
@@ -108,6 +106,7 @@ int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b
     const ResLayout &l = *mesh->res_layout(order_kind, plan.nr, this->st);   // built by the plan
     ResArgs a{};
     a.n = n;
+    a.K = nq;
     a.kc = plan.kc;
     a.nr = plan.nr;
     a.maxit = cap;
@@ -141,7 +140,7 @@ int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b
     a.x = d_x;
     a.ld = ld;
     Exec::Resident &r = e.res;
-    const int teams = (plan.K + plan.kc - 1) / plan.kc;
+    const int teams = (nq + plan.kc - 1) / plan.kc;
     const size_t elems = (size_t)n * teams * plan.kc;
     if (r.pub_p.n < elems * sin) r.pub_p.alloc(elems * sin);
     if (!cg && r.pub_s.n < elems * sin) r.pub_s.alloc(elems * sin);
@@ -167,39 +166,35 @@ int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b
     // reductions of one launch, at most: eight per iteration (replacements
     // included) and those of the replacements between iterations
     const unsigned need = (unsigned)std::min<long>(8l * cap + 8192, 0x7fffffffl);
+    if (r.epoch > 0xffffffffu - need) {
+        TMI_HIP(hipMemsetAsync(r.words.p, 0, r.words.bytes(), st));
+        r.epoch = 0;
+    }
+    a.epoch = r.epoch;
+    r.epoch += need;
+    // omegas and the cleared abort word in one upload
+    for (int c = 0; c < 64; c++) h_om[c] = mf && c < nq ? h_omega[c] : 0.0;
+    *(int *)(h_om + 64) = 0;
+    TMI_HIP(hipMemcpyAsync(d_om, h_om, sizeof(double) * 64 + 8, hipMemcpyHostToDevice, st));
+    a.omega = mf ? d_om : nullptr;
+    const bool ok = cg ? launch_resident_cg(vk, plan.cl, plan.E, bil, mf, a, lds, st)
+                       : launch_resident_bicg(vk, plan.cl, plan.E, a, lds, st);
+    if (!ok) return -1;
+    TMI_HIP(hipMemcpyAsync(r.h_ctl, r.ctl.p, r.ctl.n, hipMemcpyDeviceToHost, st));
+    TMI_HIP(hipStreamSynchronize(st));
+    e.n_sync++;
+    if (*(int *)(h_om + 64)) return -1;
+    const ResColOut *out = (const ResColOut *)r.h_ctl;
     int notconv = 0;
-    for (int q0 = 0; q0 < nq; q0 += plan.K) {
-        a.K = std::min(plan.K, nq - q0);
-        a.q0 = q0;
-        if (r.epoch > 0xffffffffu - need) {
-            TMI_HIP(hipMemsetAsync(r.words.p, 0, r.words.bytes(), st));
-            r.epoch = 0;
-        }
-        a.epoch = r.epoch;
-        r.epoch += need;
-        // omegas and the cleared abort word in one upload
-        for (int c = 0; c < 64; c++) h_om[c] = mf && c < a.K ? h_omega[q0 + c] : 0.0;
-        *(int *)(h_om + 64) = 0;
-        TMI_HIP(hipMemcpyAsync(d_om, h_om, sizeof(double) * 64 + 8, hipMemcpyHostToDevice, st));
-        a.omega = mf ? d_om : nullptr;
-        const bool ok = cg ? launch_resident_cg(vk, plan.cl, plan.E, bil, mf, a, lds, st)
-                           : launch_resident_bicg(vk, plan.cl, plan.E, a, lds, st);
-        if (!ok) return -1;
-        TMI_HIP(hipMemcpyAsync(r.h_ctl, r.ctl.p, r.ctl.n, hipMemcpyDeviceToHost, st));
-        TMI_HIP(hipStreamSynchronize(st));
-        e.n_sync++;
-        if (*(int *)(h_om + 64)) return -1;
-        const ResColOut *out = (const ResColOut *)r.h_ctl;
-        for (int c = 0; c < a.K; c++) {
-            const double b2 = out[c].bnorm2, r2 = out[c].res2;
-            const bool conv = b2 == 0.0 || r2 <= a.tol2 * b2;
-            if (!conv) notconv++;
-            stats[q0 + c].iters = out[c].iters;
-            stats[q0 + c].sweeps = out[c].sweeps;
-            stats[q0 + c].relres = b2 > 0.0 ? std::sqrt(r2 / b2) : 0.0;
-            stats[q0 + c].converged = conv ? 1 : 0;
-            e.last_iters += out[c].iters;
-        }
+    for (int c = 0; c < nq; c++) {
+        const double b2 = out[c].bnorm2, r2 = out[c].res2;
+        const bool conv = b2 == 0.0 || r2 <= a.tol2 * b2;
+        if (!conv) notconv++;
+        stats[c].iters = out[c].iters;
+        stats[c].sweeps = out[c].sweeps;
+        stats[c].relres = b2 > 0.0 ? std::sqrt(r2 / b2) : 0.0;
+        stats[c].converged = conv ? 1 : 0;
+        e.last_iters += out[c].iters;
     }
     return notconv;
 }

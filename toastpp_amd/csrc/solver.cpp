@@ -688,7 +688,7 @@ int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_co
         if (!mf) prepare_row_blocks64(sval64.p);   // the FP64 residual's operator
     };
     const ResPlan plan = resident_plan(nq, md);
-    if (plan.K == 0) row_blocks();
+    if (plan.nr == 0) row_blocks();
     std::vector<tmi_colstat> own;
     if (!stats) {
         own.resize(nq);
@@ -703,12 +703,12 @@ int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_co
     TMI_HIP(hipEventRecord(e0, es_));
     e.last_iters = 0.0;
     const long long calls0 = g_launch_calls, graphs0 = e.n_graph, syncs0 = e.n_sync;
-    int notconv = plan.K > 0 ? solve_resident(e, plan, nq, d_b, d_x, ld, stats, md, h_omega) : -1;
+    int notconv = plan.nr > 0 ? solve_resident(e, plan, nq, d_b, d_x, ld, stats, md, h_omega) : -1;
     e.res_md = notconv >= 0 ? md : -1;
     const bool sequence = notconv < 0;
     if (sequence) {
         notconv = 0;
-        if (plan.K > 0) row_blocks();   // the resident solve was refused or gave up
+        if (plan.nr > 0) row_blocks();   // the resident solve was refused or gave up
     }
     for (int q0 = 0; sequence && q0 < nq; q0 += K) {
         int kc = std::min(K, nq - q0);
@@ -949,7 +949,7 @@ void Solver::autotune(int nq, const void *d_b, void *d_x, int ld, int *tile_out,
         seq.reset();
         const unsigned long long bit = nq <= 64 ? 1ull << (nq - 1) : 0;
         tuned_sequence[mode] &= ~bit;
-        if (resident_plan(nq, mode).K > 0) {
+        if (resident_plan(nq, mode).nr > 0) {
             zero_x();
             solve(nq, d_b, d_x, ld, nullptr);   // its first run builds the layout
             zero_x();

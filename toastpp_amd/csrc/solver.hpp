@@ -182,8 +182,7 @@ struct Solver {
     int solve_tile(Exec &e, int K, int kc, tmi_colstat *stats, void *d_x, int ld, int q0, int md,
                    const double *h_omega);
     struct ResPlan {
-        int K = 0;    // columns per launch (0: the launch sequence)
-        int nr = 1;   // ranks (workgroups) per team
+        int nr = 0;   // ranks (workgroups) per team (0: the launch sequence)
         int kc = 1;   // columns per team, a power of two
         int cl = 1;   // columns per lane
         int E = 1;    // rows per thread
