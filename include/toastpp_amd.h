@@ -310,6 +310,14 @@ int tmi_solver_last_timing(tmi_solver s, double *solve_ms, double *iters_per_col
  * calls, HIP graph launches and host synchronisations (any may be NULL). */
 int tmi_solver_last_counts(tmi_solver s, long long *kernel_launches, long long *graph_launches,
                            long long *host_syncs);
+/* Whether the last CalcFields ran resident (tmi_solver_set_tile), and how many
+ * resident launches since Allocate the device refused or gave up after their
+ * bounded waits; such a block is solved by the launch sequence, and after one
+ * the handle keeps to that.  Either may be NULL. */
+int tmi_solver_last_resident(tmi_solver s, int *resident, int *given_up);
+/* For tests: what = 1 refuses the resident launches, 2 starts them with the
+ * abort word set, which ends their waits; 0: none of both. */
+int tmi_test_resident(tmi_solver s, int what);
 /* HIP graphs for the block Krylov iteration (no reference counterpart): with
  * enable = 1 (default) each check period of the BiCGSTAB / PCG iteration --
  * 8 iterations and the reliable update when it falls due, 64 to 104 kernel

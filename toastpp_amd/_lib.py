@@ -59,6 +59,8 @@ _SIGS = {
     "tmi_device_info": [C.c_char_p, C.c_int, DP],
     "tmi_synchronize": [],
     "tmi_test_alloc_limit": [C.c_double],
+    "tmi_test_resident": [P, C.c_int],
+    "tmi_solver_last_resident": [P, IP, IP],
     "tmi_device_alloc": [C.c_ulonglong, PP],
     "tmi_device_free": [P],
     "tmi_memcpy_h2d": [P, P, C.c_ulonglong],

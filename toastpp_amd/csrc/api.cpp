@@ -896,6 +896,23 @@ int tmi_solver_last_counts(tmi_solver h, long long *kernel_launches, long long *
     API_END
 }
 
+int tmi_solver_last_resident(tmi_solver h, int *resident, int *given_up)
+{
+    API_BEGIN
+    Solver &s = S(h);
+    if (resident) *resident = s.ex.res_md >= 0 ? 1 : 0;
+    if (given_up) *given_up = s.res_given_up;
+    API_END
+}
+
+int tmi_test_resident(tmi_solver h, int what)
+{
+    API_BEGIN
+    TMI_CHECK(what >= 0 && what <= 2, TMI_ERR_INVALID_ARG, "unknown test %d", what);
+    S(h).test_resident = what;
+    API_END
+}
+
 int tmi_solver_set_graphs(tmi_solver h, int enable)
 {
     API_BEGIN

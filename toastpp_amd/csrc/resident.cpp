@@ -33,7 +33,7 @@ Solver::ResPlan Solver::resident_plan(int nq, int md)
     const VKind vk = mixed ? vk32() : vk64();
     const size_t sz = vbytes(vk);
     const bool wide = vk == VK_C64;
-    if (named || tuning || lsolver == TMI_LSOLVER_GMRES || nq < 1 || nq > 64) return none;
+    if (named || tuning || res_given_up || lsolver == TMI_LSOLVER_GMRES || nq < 1 || nq > 64) return none;
     if (tuned_sequence[md] >> (nq - 1) & 1) return none;
     if ((size_t)mesh->n * nq * sz > RES_MAX_BYTES) return none;
     int pow = 1;
@@ -90,9 +90,10 @@ const void *Solver::sliced(OpKind k, const ResLayout &l, int nr)
 }
 
 // Columns 0 .. nq-1 in one cooperative launch.  Returns the number of columns
-// above the tolerance, or -1 when the launch was refused or gave up (the
-// fields then hold initial guesses or solutions, a valid start for the launch
-// sequence).
+// above the tolerance, or -1 when the launch was refused or gave up: its
+// memory is then free again, the fields hold initial guesses or solutions, a
+// valid start for the launch sequence, and the handle keeps to that one (a
+// give-up costs the 4 s of its bounded waits).
 int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld,
                            tmi_colstat *stats, int md, const double *h_omega)
 {
@@ -174,16 +175,21 @@ int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b
     r.epoch += need;
     // omegas and the cleared abort word in one upload
     for (int c = 0; c < 64; c++) h_om[c] = mf && c < nq ? h_omega[c] : 0.0;
-    *(int *)(h_om + 64) = 0;
+    *(int *)(h_om + 64) = test_resident == 2 ? 1 : 0;
     TMI_HIP(hipMemcpyAsync(d_om, h_om, sizeof(double) * 64 + 8, hipMemcpyHostToDevice, st));
     a.omega = mf ? d_om : nullptr;
-    const bool ok = cg ? launch_resident_cg(vk, plan.cl, plan.E, bil, mf, a, lds, st)
-                       : launch_resident_bicg(vk, plan.cl, plan.E, a, lds, st);
-    if (!ok) return -1;
-    TMI_HIP(hipMemcpyAsync(r.h_ctl, r.ctl.p, r.ctl.n, hipMemcpyDeviceToHost, st));
-    TMI_HIP(hipStreamSynchronize(st));
-    e.n_sync++;
-    if (*(int *)(h_om + 64)) return -1;
+    const bool ok = test_resident != 1 && (cg ? launch_resident_cg(vk, plan.cl, plan.E, bil, mf, a, lds, st)
+                                              : launch_resident_bicg(vk, plan.cl, plan.E, a, lds, st));
+    if (ok) {
+        TMI_HIP(hipMemcpyAsync(r.h_ctl, r.ctl.p, r.ctl.n, hipMemcpyDeviceToHost, st));
+        TMI_HIP(hipStreamSynchronize(st));
+        e.n_sync++;
+    }
+    if (!ok || *(int *)(h_om + 64)) {
+        res_given_up++;
+        e.release_resident();
+        return -1;
+    }
     const ResColOut *out = (const ResColOut *)r.h_ctl;
     int notconv = 0;
     for (int c = 0; c < nq; c++) {

@@ -119,14 +119,20 @@ void Solver::Exec::release_work()
             w.oic.release();
             w.K = w.n = w.G = 0;
         }
+    release_resident();
+    free_gmres_work(gm);
+    gm = nullptr;
+}
+
+void Solver::Exec::release_resident()
+{
+    if (st) TMI_HIP(hipStreamSynchronize(st));
     res.pub_p.release();
     res.pub_s.release();
     res.rd0.release();
     res.x64.release();
     res.words.release();   // cleared again before the next use
     res.ctl.release();
-    free_gmres_work(gm);
-    gm = nullptr;
 }
 
 void Solver::allocate()
@@ -138,6 +144,7 @@ void Solver::allocate()
     sval32.alloc(nval() + 8);   // + 16-byte-chunk slack for the LDS-DMA SpMM's value staging
     allocated = true;
     assembled = false;
+    res_given_up = 0;
 }
 
 BlockDesc Solver::block(const Exec::Work &w, int K) const
@@ -672,7 +679,10 @@ int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_co
         std::lock_guard<std::mutex> lk(prep_mu);
         prepare_mf();
     }
-    if (lsolver == TMI_LSOLVER_GMRES) return gmres_on(e, nq, d_b, d_x, ld, stats);
+    if (lsolver == TMI_LSOLVER_GMRES) {
+        e.res_md = -1;
+        return gmres_on(e, nq, d_b, d_x, ld, stats);
+    }
     if (precon == TMI_PRECON_DIAG) {
         std::lock_guard<std::mutex> lk(prep_mu);
         if (!precon_valid) {
@@ -704,7 +714,6 @@ int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_co
     e.last_iters = 0.0;
     const long long calls0 = g_launch_calls, graphs0 = e.n_graph, syncs0 = e.n_sync;
     int notconv = plan.nr > 0 ? solve_resident(e, plan, nq, d_b, d_x, ld, stats, md, h_omega) : -1;
-    e.res_md = notconv >= 0 ? md : -1;
     const bool sequence = notconv < 0;
     if (sequence) {
         notconv = 0;
@@ -768,6 +777,7 @@ int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_co
     (void)hipEventDestroy(e1);
     e.last_solve_ms = ms;
     e.last_iters = nq ? iters / nq : 0.0;
+    e.res_md = sequence ? -1 : md;   // (an FP64 fallback has set its own)
     return notconv;
 }
 

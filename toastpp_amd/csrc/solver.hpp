@@ -1,5 +1,6 @@
 // Forward solver: the GPU counterpart of TFwdSolver<T> (fwdsolver.h:77-508).
 #pragma once
+#include <atomic>
 #include <cstdlib>
 #include <mutex>
 
@@ -97,6 +98,7 @@ struct Solver {
             char *h_ctl = nullptr;
         } res;
         int res_md = -1;               // mode of the last solve, if it ran resident
+        void release_resident();       // free what resident solves hold
         GmresWork *gm = nullptr;       // GMRES workspace (allocated by the first GMRES solve)
         double last_solve_ms = 0.0, last_iters = 0.0;
         // instantiated graphs of the check period's launch sequence, keyed by
@@ -129,6 +131,10 @@ struct Solver {
     // ... as do those the autotuner found it faster for: per mode, bit nq - 1
     unsigned long long tuned_sequence[3] = {0, 0, 0};
     bool tuning = false;   // the autotuner is timing the launch sequence
+    // resident launches that were refused or gave up since Allocate: after one
+    // the handle keeps to the launch sequence
+    std::atomic<int> res_given_up{0};
+    int test_resident = 0;   // tests: 1 refuse the launch, 2 start with the abort word set
 
     ~Solver();
     VKind vk64() const { return cplx ? VK_C64 : VK_R64; }

@@ -235,6 +235,13 @@ class FwdSolver:
         L.call("tmi_solver_last_counts", self._h, C.byref(k), C.byref(g), C.byref(s))
         return k.value, g.value, s.value
 
+    def LastResident(self):
+        """(whether the last CalcFields ran resident, resident launches that
+        were refused or gave up since Allocate)"""
+        r, g = C.c_int(), C.c_int()
+        L.call("tmi_solver_last_resident", self._h, C.byref(r), C.byref(g))
+        return bool(r.value), g.value
+
     def LastTiming(self):
         ms, it = C.c_double(), C.c_double()
         L.call("tmi_solver_last_timing", self._h, C.byref(ms), C.byref(it))
