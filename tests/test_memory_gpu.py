@@ -48,3 +48,22 @@ def test_solve_after_out_of_memory(limit, solver):
         assert e.value.code == L.TMI_ERR_OOM
     limit(0)
     assert np.array_equal(_fields(f, B), ref)
+
+
+@pytest.mark.parametrize("limit_bytes", [20000, 1519 * 16 * 8 - 1])
+def test_resident_solve_without_memory(limit, limit_bytes):
+    """Where the resident layout (20 KB: less than it takes) or the vectors of
+    all columns find no memory, the launch sequence solves one right-hand side
+    after the other."""
+    mesh, f, B = _prepared("BICGSTAB", False)
+    f.SetMode("fp64")
+    f.SetTile(1)
+    ref = _fields(f, B)   # the launch sequence has its workspace from here on
+    f.SetTile(0)
+    dB, dX = L.DeviceArray.from_host(B), L.DeviceArray(B.shape, B.dtype)
+    limit(limit_bytes)
+    f.CalcFieldsDevice(16, dB.ptr, dX.ptr)
+    assert f.LastResident() == (False, 0) and np.array_equal(dX.to_host(), ref)
+    limit(0)
+    f.CalcFieldsDevice(16, dB.ptr, dX.ptr)
+    assert f.LastResident() == (True, 0)

@@ -53,7 +53,13 @@ Solver::ResPlan Solver::resident_plan(int nq, int md)
         // instantiations (krylov_resident_*.hip)
         const int emax = cl == 1 ? (wide && bicg ? 4 : 8) : (bicg ? 2 : 4);
         if (E > emax) continue;   // fewer, longer teams
-        const ResLayout *l = mesh->res_layout(order_kind, nr, st);
+        const ResLayout *l = nullptr;
+        try {
+            l = mesh->res_layout(order_kind, nr, st);
+        } catch (const Error &err) {
+            if (err.code != TMI_ERR_OOM) throw;
+            return none;   // the launch sequence needs none
+        }
         if (!l || l->nu == INT_MAX) continue;
         if ((((size_t)l->nu * kc * sz + 15) & ~(size_t)15) + res_lds_fixed(kc) > RES_LDS) continue;
         ResPlan p;
@@ -89,13 +95,27 @@ const void *Solver::sliced(OpKind k, const ResLayout &l, int nr)
     return o.v.p;
 }
 
+// As below, and -1 when there is no memory for it (the launch sequence works in
+// narrower tiles, or has its own already)
+int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld,
+                           tmi_colstat *stats, int md, const double *h_omega)
+{
+    try {
+        return launch_resident(e, plan, nq, d_b, d_x, ld, stats, md, h_omega);
+    } catch (const Error &err) {
+        if (err.code != TMI_ERR_OOM) throw;
+        e.release_resident();
+        return -1;
+    }
+}
+
 // Columns 0 .. nq-1 in one cooperative launch.  Returns the number of columns
 // above the tolerance, or -1 when the launch was refused or gave up: its
 // memory is then free again, the fields hold initial guesses or solutions, a
 // valid start for the launch sequence, and the handle keeps to that one (a
 // give-up costs the 4 s of its bounded waits).
-int Solver::solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld,
-                           tmi_colstat *stats, int md, const double *h_omega)
+int Solver::launch_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld,
+                            tmi_colstat *stats, int md, const double *h_omega)
 {
     hipStream_t st = e.st;
     const int n = mesh->n;

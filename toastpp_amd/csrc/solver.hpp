@@ -197,6 +197,8 @@ struct Solver {
     static size_t resident_fixed_bytes();   // words and results, whatever the block
     int solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats,
                        int md, const double *h_omega);
+    int launch_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats,
+                        int md, const double *h_omega);
     // operators in the slice order of a resident layout, per operator kind
     // and number of ranks; valid until the next assembly
     enum OpKind { OPK_32, OPK_64, OPK_P32, OPK_P64, OPK_MF32, OPK_MF64, OPK_N };
