@@ -26,16 +26,21 @@ static constexpr size_t RES_MAX_BYTES = 8500000;
 static constexpr long RES_MAX_ENTRIES = 8000000;
 static constexpr int RES_ONE_WG = 1500;
 
+bool Solver::resident_block(int nq, int md) const
+{
+    if (named || tuning || res_given_up || lsolver == TMI_LSOLVER_GMRES || nq < 1 || nq > 64) return false;
+    if (tuned_sequence[md] >> (nq - 1) & 1) return false;
+    return (size_t)mesh->n * nq * vbytes(md == TMI_MODE_MIXED_BLOCK ? vk32() : vk64()) <= RES_MAX_BYTES;
+}
+
 Solver::ResPlan Solver::resident_plan(int nq, int md)
 {
     ResPlan none;
+    if (!resident_block(nq, md)) return none;
     const bool mixed = md == TMI_MODE_MIXED_BLOCK, bicg = !pcg();
     const VKind vk = mixed ? vk32() : vk64();
     const size_t sz = vbytes(vk);
     const bool wide = vk == VK_C64;
-    if (named || tuning || res_given_up || lsolver == TMI_LSOLVER_GMRES || nq < 1 || nq > 64) return none;
-    if (tuned_sequence[md] >> (nq - 1) & 1) return none;
-    if ((size_t)mesh->n * nq * sz > RES_MAX_BYTES) return none;
     int pow = 1;
     while (pow < nq) pow *= 2;
     int T = mesh->n <= RES_ONE_WG ? RES_WG : pow;
@@ -71,9 +76,19 @@ Solver::ResPlan Solver::resident_plan(int nq, int md)
     }
 }
 
-size_t Solver::resident_fixed_bytes()
+static constexpr size_t RES_CTL_BYTES = sizeof(ResColOut) * 64 + sizeof(double) * 64 + 8;
+
+// Vectors of the columns rounded up to whole teams (a power of two at most),
+// words and results
+size_t Solver::resident_bytes(int nq, int md) const
 {
-    return (RES_PART_WORDS + RES_TOT_WORDS) * sizeof(res_u64) + sizeof(ResColOut) * 64 + sizeof(double) * 64 + 8;
+    if (!resident_block(nq, md)) return 0;
+    const bool mixed = md == TMI_MODE_MIXED_BLOCK;
+    const size_t sin = vbytes(mixed ? vk32() : vk64()), inner = pcg() ? 1 : mixed ? 2 : 3;
+    size_t cols = 1;
+    while (cols < (size_t)nq) cols *= 2;
+    return mesh->n * cols * (inner * sin + vbytes(vk64())) + (RES_PART_WORDS + RES_TOT_WORDS) * sizeof(res_u64) +
+           RES_CTL_BYTES;
 }
 
 const void *Solver::sliced(OpKind k, const ResLayout &l, int nr)
@@ -171,7 +186,7 @@ int Solver::launch_resident(Exec &e, const ResPlan &plan, int nq, const void *d_
         r.words.alloc(RES_PART_WORDS + RES_TOT_WORDS);
         r.epoch = 0xffffffffu;   // cleared below before the first use
     }
-    if (!r.ctl.p) r.ctl.alloc(sizeof(ResColOut) * 64 + sizeof(double) * 64 + 8);
+    if (!r.ctl.p) r.ctl.alloc(RES_CTL_BYTES);
     if (!r.h_ctl) TMI_HIP(hipHostMalloc((void **)&r.h_ctl, r.ctl.n));
     double *d_om = (double *)(r.ctl.p + sizeof(ResColOut) * 64);
     double *h_om = (double *)(r.h_ctl + sizeof(ResColOut) * 64);

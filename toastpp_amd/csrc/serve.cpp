@@ -36,6 +36,7 @@ struct ServeRequest {
     const void *d_b = nullptr;
     void *d_x = nullptr;
     size_t bytes = 0;
+    bool resident = true;   // false: the budget holds the launch sequence's workspace only
     double t_queued = 0, t_started = 0, t_finished = 0;
     int status = TMI_OK;
     bool done = false;
@@ -73,6 +74,10 @@ class Server {
         r->d_b = d_b;
         r->d_x = d_x;
         r->bytes = s->work_bytes(nq);
+        if ((double)r->bytes > budget_) {
+            r->resident = false;
+            r->bytes = s->work_bytes(nq, false);
+        }
         TMI_CHECK((double)r->bytes <= budget_, TMI_ERR_OOM,
                   "request needs %.1f MiB of workspace, more than the server's HBM budget", r->bytes / 1048576.0);
         r->t_queued = now();
@@ -156,7 +161,8 @@ class Server {
             }
             r->stats.assign(r->nq, tmi_colstat{});
             try {
-                int nc = r->solver->solve_on(e, r->nq, r->d_b, r->d_x, r->ld, r->stats.data());
+                int nc = r->solver->solve_on(e, r->nq, r->d_b, r->d_x, r->ld, r->stats.data(), -1, nullptr,
+                                             r->resident);
                 r->status = nc ? TMI_ERR_NOT_CONVERGED : TMI_OK;
             } catch (const Error &ex) {
                 r->status = ex.code;

@@ -83,24 +83,33 @@ int Solver::tile_for(int nq, int md) const
     return K;
 }
 
-size_t Solver::work_bytes(int nq) const
+size_t Solver::work_bytes(int nq, bool resident) const
 {
     if (lsolver == TMI_LSOLVER_GMRES) return gmres_tile_bytes(mesh->n, tile_for(nq, TMI_MODE_FP64_BLOCK), vbytes(vk64()));
     // the tile and, with compaction, its narrower copies (K/2 + K/4 + ... < K)
-    // and the second workspaces of the repacked widths (K and K/2)
-    const size_t K = tile_for(nq), n = mesh->n, Kall = compact_min > 0 ? 2 * K + K + K / 2 : K;
-    const bool mixed = mode == TMI_MODE_MIXED_BLOCK;
+    // and the second workspaces of the repacked widths (K and K/2); without it,
+    // the FP64 fallback of fewer columns may take a narrower one beside it
+    const bool mixed = mode == TMI_MODE_MIXED_BLOCK, fallback = mixed && fp64_fallback;
+    const size_t K = tile_for(nq), n = mesh->n;
+    const size_t Kall = compact_min > 0 ? 2 * K + K + K / 2 : fallback ? K + K / 2 : K;
     const size_t s64 = vbytes(vk64()), sin = vbytes(mixed ? vk32() : vk64());
     auto tiles = [&](size_t s_inner) {
         return n * Kall * (3 * s64 + 7 * s_inner) + RED_SLOTS * 2048 * Kall * 8 + (S_NSLOT * 2 * 8 + I_NSLOT * 2 * 4) * Kall;
     };
     size_t b = tiles(sin);
     if (mixed && K == 64 && cplx) b += 2 * n * 32;   // packed shadow residuals (both 64-column workspaces)
+    // a resident solve instead (one that gives up frees its vectors first)
+    const size_t res = resident ? resident_bytes(nq, mode) : 0;
+    if (!fallback) return std::max(b, res);
     // the FP64 fallback of the mixed mode re-solves unconverged columns in
-    // FP64: the workspaces it uses are reallocated with FP64 inner vectors,
-    // and their right-hand sides and solutions are copied (at most nq each)
-    if (mixed && fp64_fallback) b = std::max(b, tiles(s64)) + 2 * n * (size_t)nq * s64;
-    return b + resident_fixed_bytes();   // (its vectors take less than the tiles')
+    // FP64, beside what the first solve holds: tile workspaces are reallocated
+    // with FP64 inner vectors, resident vectors are added to the tiles or the
+    // other way round, and the right-hand sides and solutions are copied (at
+    // most nq each)
+    size_t res64 = 0;
+    if (resident)
+        for (int nb = 1; nb <= std::min(nq, 64); nb++) res64 = std::max(res64, resident_bytes(nb, TMI_MODE_FP64_BLOCK));
+    return std::max({b, tiles(s64), b + res64, res + tiles(s64), res + res64}) + 2 * n * (size_t)nq * s64;
 }
 
 void Solver::Exec::release_work()
@@ -660,7 +669,7 @@ void Solver::prepare_row_blocks(const float *op)
 }
 
 int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats, int md,
-                     const double *h_omega)
+                     const double *h_omega, bool resident)
 {
     TMI_CHECK(assembled, TMI_ERR_STATE, "CalcFields called before Reset/AssembleSystemMatrix");
     TMI_CHECK(!(cplx && lsolver == TMI_LSOLVER_CG), TMI_ERR_UNSUPPORTED,
@@ -697,7 +706,7 @@ int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_co
         prepare_row_blocks(mf ? mfval32.p : spmm_op32());
         if (!mf) prepare_row_blocks64(sval64.p);   // the FP64 residual's operator
     };
-    const ResPlan plan = resident_plan(nq, md);
+    const ResPlan plan = resident ? resident_plan(nq, md) : ResPlan{};
     if (plan.nr == 0) row_blocks();
     std::vector<tmi_colstat> own;
     if (!stats) {
@@ -749,7 +758,8 @@ int Solver::solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_co
         std::vector<double> om2;
         if (mf)
             for (int j = 0; j < nb; j++) om2.push_back(h_omega[bad[j]]);
-        solve_on(e, nb, tb.p, tx.p, nb, st2.data(), TMI_MODE_FP64_BLOCK, mf ? om2.data() : nullptr);
+        solve_on(e, nb, tb.p, tx.p, nb, st2.data(), TMI_MODE_FP64_BLOCK, mf ? om2.data() : nullptr,
+                 resident);
         iters += e.last_iters * nb;
         notconv = 0;
         for (int j = 0; j < nb; j++) {

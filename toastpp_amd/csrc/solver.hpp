@@ -153,9 +153,10 @@ struct Solver {
     // h_omega (host, nq values, complex COCG, block modes): column c solves
     // at omega h_omega[c] -- several frequencies in one block solve
     int solve_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats, int md = -1,
-                 const double *h_omega = nullptr);
-    // device bytes a solve of nq columns needs for its workspace
-    size_t work_bytes(int nq) const;
+                 const double *h_omega = nullptr, bool resident = true);
+    // device bytes a solve of nq columns needs for its workspace (resident
+    // false: by the launch sequence, as solve_on with the same argument)
+    size_t work_bytes(int nq, bool resident = true) const;
     int tile_for(int nq, int md = -1) const;
     // replay the check period's launches from captured HIP graphs (default
     // on; the environment variable TMI_GRAPHS=0 turns it off for new solvers,
@@ -194,7 +195,8 @@ struct Solver {
         int E = 1;    // rows per thread
     };
     ResPlan resident_plan(int nq, int md);
-    static size_t resident_fixed_bytes();   // words and results, whatever the block
+    bool resident_block(int nq, int md) const;     // whether its size and the handle's settings allow it
+    size_t resident_bytes(int nq, int md) const;   // device bytes of a resident solve, at most
     int solve_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats,
                        int md, const double *h_omega);
     int launch_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats,
