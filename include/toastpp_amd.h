@@ -315,6 +315,11 @@ int tmi_solver_last_counts(tmi_solver s, long long *kernel_launches, long long *
  * bounded waits; such a block is solved by the launch sequence, and after one
  * the handle keeps to that.  Either may be NULL. */
 int tmi_solver_last_resident(tmi_solver s, int *resident, int *given_up);
+/* Device bytes of the operators' copies in the order of resident solves, which
+ * the handle keeps beside the workspaces tmi_solver_work_bytes counts: one per
+ * operator and number of workgroups a block takes, the least recently used
+ * given back above 256 MiB (or what one solve needs). */
+int tmi_solver_operator_bytes(tmi_solver s, double *bytes);
 /* For tests: what = 1 refuses the resident launches, 2 starts them with the
  * abort word set, which ends their waits; 0: none of both. */
 int tmi_test_resident(tmi_solver s, int what);
@@ -345,7 +350,9 @@ int tmi_jacobian_nodal(tmi_mesh m, int nq, int nm, const double *dphi, const dou
 /* Same on GPU-resident arrays: d_dphi nlen rows of ldd complex (first nq
  * used), d_aphi nlen rows of lda complex (first nm used), so that direct and
  * adjoint fields of one block solve can be passed in place; d_J must hold
- * 4 nqm nlen doubles. */
+ * 4 nqm nlen doubles.  The first nodal Jacobian of a mesh makes the nodes'
+ * element-integral matrices, which the mesh keeps until it is freed: 4 KB a
+ * node (16 KB where rows have more than 16 entries), at most 1 GiB. */
 int tmi_jacobian_nodal_device(tmi_mesh m, int nq, int nm, const void *d_dphi, int ldd, const void *d_aphi,
                               int lda, const void *d_proj, int dscale, void *d_J);
 /* GenerateJacobian_cw, nodal basis (jacobian.cc:132-186 with raster ==

@@ -60,6 +60,7 @@ _SIGS = {
     "tmi_synchronize": [],
     "tmi_test_alloc_limit": [C.c_double],
     "tmi_test_resident": [P, C.c_int],
+    "tmi_solver_operator_bytes": [P, DP],
     "tmi_solver_last_resident": [P, IP, IP],
     "tmi_device_alloc": [C.c_ulonglong, PP],
     "tmi_device_free": [P],

@@ -905,6 +905,16 @@ int tmi_solver_last_resident(tmi_solver h, int *resident, int *given_up)
     API_END
 }
 
+int tmi_solver_operator_bytes(tmi_solver h, double *bytes)
+{
+    API_BEGIN
+    NEED(bytes);
+    Solver &s = S(h);
+    std::lock_guard<std::mutex> lk(s.prep_mu);
+    *bytes = (double)s.slice_bytes();
+    API_END
+}
+
 int tmi_test_resident(tmi_solver h, int what)
 {
     API_BEGIN

@@ -91,7 +91,7 @@ size_t Solver::resident_bytes(int nq, int md) const
            RES_CTL_BYTES;
 }
 
-const void *Solver::sliced(OpKind k, const ResLayout &l, int nr)
+Solver::Slices Solver::sliced(OpKind k, const ResLayout &l, int nr)
 {
     int lg = 0;
     while ((1 << lg) < nr) lg++;
@@ -101,13 +101,39 @@ const void *Solver::sliced(OpKind k, const ResLayout &l, int nr)
                     : k == OPK_P32 ? (const void *)pval32.p : k == OPK_P64 ? (const void *)pval64.p
                     : k == OPK_MF32 ? (const void *)mfval32.p : (const void *)mfval64.p;
     const size_t es = (f32 ? 4 : 8) * (cplx ? 2 : 1);
+    o.used = slice_clock;
     if (!o.valid) {
-        o.v.alloc((size_t)l.nent * es);
-        launch_slice_vals((int)es, l.nent, l.slot.p, src, o.v.p, st);
+        if (!o.v || o.v->bytes() != (size_t)l.nent * es) {
+            o.v.reset();
+            o.v = std::make_shared<DBuf<char>>((size_t)l.nent * es);
+        }
+        launch_slice_vals((int)es, l.nent, l.slot.p, src, o.v->p, st);
         TMI_HIP(hipStreamSynchronize(st));   // other streams read it next
         o.valid = true;
     }
-    return o.v.p;
+    return o.v;
+}
+
+size_t Solver::slice_bytes() const
+{
+    size_t b = 0;
+    for (auto &k : slice_op)
+        for (const SliceOp &o : k) b += o.v ? o.v->bytes() : 0;
+    return b;
+}
+
+void Solver::trim_slices()
+{
+    for (size_t held = slice_bytes(); held > SLICE_BYTES;) {
+        SliceOp *old = nullptr;
+        for (auto &k : slice_op)
+            for (SliceOp &o : k)
+                if (o.v && o.used != slice_clock && (!old || o.used < old->used)) old = &o;
+        if (!old) return;
+        held -= old->v->bytes();
+        old->v.reset();   // freed with the last solve that holds it
+        old->valid = false;
+    }
 }
 
 // As below, and -1 when there is no memory for it (the launch sequence works in
@@ -161,13 +187,18 @@ int Solver::launch_resident(Exec &e, const ResPlan &plan, int nq, const void *d_
     a.halo = l.halo.p;
     a.lcol = l.lcol.p;
     a.gcol = l.gcol.p;
+    Slices op, op64;   // held until the launch has ended
     {
         std::lock_guard<std::mutex> lk(prep_mu);
+        slice_clock++;
         const bool right = diag && !cg;   // BiCGSTAB iterates with K D^-1
-        a.op = sliced(mf ? (mixed ? OPK_MF32 : OPK_MF64)
+        op = sliced(mf ? (mixed ? OPK_MF32 : OPK_MF64)
                          : right ? (mixed ? OPK_P32 : OPK_P64) : (mixed ? OPK_32 : OPK_64), l, plan.nr);
-        a.op64 = (const double *)sliced(mf ? OPK_MF64 : OPK_64, l, plan.nr);
+        op64 = sliced(mf ? OPK_MF64 : OPK_64, l, plan.nr);
+        trim_slices();
     }
+    a.op = op->p;
+    a.op64 = (const double *)op64->p;
     if (diag) {
         if (mf) a.idiag = mixed ? (const void *)mfdiag32.p : (const void *)mfdiag64.p;
         else a.idiag = mixed ? (const void *)idiag32.p : (const void *)idiag64.p;

@@ -1,6 +1,7 @@
 // Forward solver: the GPU counterpart of TFwdSolver<T> (fwdsolver.h:77-508).
 #pragma once
 #include <atomic>
+#include <memory>
 #include <cstdlib>
 #include <mutex>
 
@@ -157,6 +158,7 @@ struct Solver {
     // device bytes a solve of nq columns needs for its workspace (resident
     // false: by the launch sequence, as solve_on with the same argument)
     size_t work_bytes(int nq, bool resident = true) const;
+    size_t slice_bytes() const;   // ... held for operators in slice order (caller holds prep_mu)
     int tile_for(int nq, int md = -1) const;
     // replay the check period's launches from captured HIP graphs (default
     // on; the environment variable TMI_GRAPHS=0 turns it off for new solvers,
@@ -202,13 +204,21 @@ struct Solver {
     int launch_resident(Exec &e, const ResPlan &plan, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats,
                         int md, const double *h_omega);
     // operators in the slice order of a resident layout, per operator kind
-    // and number of ranks; valid until the next assembly
+    // and number of ranks; valid until the next assembly.  Blocks of other
+    // sizes take other numbers of ranks: up to SLICE_BYTES of copies are kept
+    // (or what one solve needs), then the least recently used go; a solve
+    // holds its own until it has ended.
     enum OpKind { OPK_32, OPK_64, OPK_P32, OPK_P64, OPK_MF32, OPK_MF64, OPK_N };
+    static constexpr size_t SLICE_BYTES = (size_t)256 << 20;
+    using Slices = std::shared_ptr<DBuf<char>>;
     struct SliceOp {
-        DBuf<char> v;
+        Slices v;
         bool valid = false;
+        unsigned long long used = 0;   // slice_clock of its last solve
     } slice_op[OPK_N][9];
-    const void *sliced(OpKind k, const ResLayout &l, int nr);   // caller holds prep_mu
+    unsigned long long slice_clock = 0;
+    Slices sliced(OpKind k, const ResLayout &l, int nr);   // caller holds prep_mu
+    void trim_slices();                                    // ... down to SLICE_BYTES, but for this clock's
     // GMRES(20) in FP64 on tiles of the columns (gmres.hip); every mode
     int gmres_on(Exec &e, int nq, const void *d_b, void *d_x, int ld, tmi_colstat *stats);
     int count_active(Exec &e, const int *d_flags, int K);

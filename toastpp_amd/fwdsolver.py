@@ -223,6 +223,12 @@ class FwdSolver:
         L.call("tmi_solver_work_bytes", self._h, int(nq), C.byref(b))
         return b.value
 
+    def OperatorBytes(self):
+        """device bytes of the operators' copies kept for resident solves"""
+        b = C.c_double()
+        L.call("tmi_solver_operator_bytes", self._h, C.byref(b))
+        return b.value
+
     def SetGraphs(self, enable=True):
         """replay the block iteration's check periods from captured HIP graphs
         (default) or launch every kernel"""
