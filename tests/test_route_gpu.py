@@ -70,3 +70,46 @@ def test_autotune_decides_for_its_own_columns(disk):
     f.SetGraphs(True)
     f.Autotune(12, dB.ptr, dX.ptr, ld=64)
     assert not _resident(f, disk, 12)
+
+
+def test_long_blocks_take_the_launch_sequence():
+    """COCG in FP32 above 16 columns: the shorter operator runs resident, the
+    longer one by the launch sequence, which is faster there."""
+    for (nodes, el), nq, resident in ((G.disk(25.0, 40), 33, True), (G.cylinder(25.0, 50.0, 20, 24), 16, True),
+                                      (G.cylinder(25.0, 50.0, 20, 24), 33, False)):
+        mesh = T.Mesh(data=(nodes, el))
+        Q = G.ring(nq, 25.0) if nodes.shape[1] == 2 else G.ring(nq, 25.0, 5.0)
+        mesh.SetQM(Q, Q[:1])
+        f = _solver((mesh, T.Solution(*G.params(nodes, 7)), None))
+        B = np.ascontiguousarray(mesh.Qvec(width=2.0).toarray())
+        dB, dX = L.DeviceArray.from_host(B), L.DeviceArray(B.shape, B.dtype)
+        f.CalcFieldsDevice(nq, dB.ptr, dX.ptr)
+        assert f.LastResident() == (resident, 0)
+
+
+@pytest.mark.parametrize("solver,mode,nq", [("BICGSTAB", "fp64_block", 4), ("BICGSTAB", "fp64", 3), ("COCG", "fp64_block", 7),
+                                            ("COCG", "mixed", 8), ("BICGSTAB", "mixed", 8), ("COCG", "mixed", 3)])
+def test_few_teams_on_many_rows(solver, mode, nq):
+    """67,951 nodes, where a thread of a team with one column would hold more
+    rows than it should: the columns share teams.  Against the launch sequence;
+    strongly absorbing tissue, so that the fields follow the residual (20 x
+    1e-10 as for the small meshes)."""
+    nodes, el = G.disk(25.0, 150)
+    mesh = T.Mesh(data=(nodes, el))
+    mesh.SetQM(G.ring(8, 25.0), G.ring(1, 25.0))
+    mua, mus, ref = G.params(nodes, 7)
+    B = np.ascontiguousarray(mesh.Qvec(width=2.0).toarray()[:, :nq])
+    X = []
+    for sequence in (False, True):
+        f = T.FwdSolver(mesh, solver, 1e-10)
+        f.SetMode(mode)
+        f.SetPrecon("DIAG")
+        if sequence:
+            f.SetGraphs(True)
+        f.Allocate()
+        f.Reset(T.Solution(100.0 * mua, mus, ref), 100.0 * 2 * np.pi * 1e-6)
+        dB, dX = L.DeviceArray.from_host(B), L.DeviceArray(B.shape, B.dtype)
+        assert all(s[3] for s in f.CalcFieldsDevice(nq, dB.ptr, dX.ptr))
+        assert f.LastResident() == (not sequence, 0)
+        X.append(dX.to_host())
+    assert (np.linalg.norm(X[0] - X[1], axis=0) / np.linalg.norm(X[1], axis=0)).max() <= 20e-10

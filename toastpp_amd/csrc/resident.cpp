@@ -14,16 +14,35 @@ namespace tmi {
 //   n 3,169 real x 16: 7.5 / 31       n 31,525 c64 x 2 (BiCGSTAB): 24 / 97
 //   n 19,441 c32 x 24: 26 / 38        n 31,525 c64 x 16: 27 / 59
 //   n 31,525 c32 x 8: 24 / 39         n 103,267 c32 x 8: 42 / 54
-//   n 31,525 c32 x 32 (BiCGSTAB): 74 / 76    n 31,525 c32 x 64: 73 / 72
-// so it is taken for blocks of up to RES_MAX_BYTES.
+//   n 31,525 c32 x 32 (BiCGSTAB): 75 / 75    n 250,047 c32 x 4: 49 / 58
+// so it is taken for blocks of up to RES_MAX_BYTES.  Above 16 columns the
+// launch sequence's complex FP32 tiles run on the matrix cores; with COCG it is
+// then the faster one for long operators (n 31,525 x 33: 79 / 71, n 50,653 x 17:
+// 65 / 55, n 39,304 x 24: 52 / 52, n 19,683 x 52: 47 / 39 but 12 % faster in all):
+// beyond RES_MAX_MACS entries times columns, rounded up to whole teams.
 static constexpr size_t RES_MAX_BYTES = 8500000;
+static constexpr long RES_MAX_MACS = 20000000;
 // Teams: one column per team keeps the reductions small and the ranks few
 // (n 19,441 x 24: 8 ranks 26 us, 32 ranks 28; n 31,525 c64 x 16: 16 ranks 27,
 // 32 ranks 34) but every team reads the matrix: beyond RES_MAX_ENTRIES
 // entries per iteration (n 103,267 x 8: 4 teams 53 us, 1 team 42) the columns
-// share as few teams as hold them.  Tiny systems run on single workgroups
-// without any exchange (n 817 x 4: 7.0 us, 4 ranks 9.4; n 3,169 x 16: 11.2).
+// share as few teams as hold them.  So they do where a thread of a team with
+// one column would hold too many rows, as most of their operator then comes
+// from memory between uses (us: one column a team / few teams / launch sequence):
+//   more than 4 rows, complex (with COCG, if the XCDs fetch more than
+//   RES_XCD_ENTRIES entries an iteration, a team of up to 32 ranks on one XCD):
+//     c32 COCG      n 132,651 x 4: 47 / 36 / 45    n 67,951 x 8: 36 / 28 / 41
+//                   n 19,441 x 24 (1.1 M entries): 25 / 28 / 37
+//     c32 BiCGSTAB  n 132,651 x 4: 97 / 64 / 69    n 19,441 x 24: 54 / 42 / 55
+//     c64 COCG      n 132,651 x 4: 77 / 44 / 54    n 67,951 x 7: 58 / 34 / 47
+//   more than 2 rows, c64 BiCGSTAB, four teams at most (each on several XCDs
+//   in any case) or twice RES_XCD_ENTRIES:
+//     n 103,267 x 4: 100 / 63 / 75    n 250,047 x 2: 112 / 75 / 104
+//     n 50,653 x 8: 81 / 60 / 70      n 31,525 x 16 (3.6 M entries): 67 / 68 / 113
+// Tiny systems run on single workgroups without any exchange (n 817 x 4: 7.0
+// us, 4 ranks 9.4; n 3,169 x 16: 11.2).
 static constexpr long RES_MAX_ENTRIES = 8000000;
+static constexpr long RES_XCD_ENTRIES = 2000000;
 static constexpr int RES_ONE_WG = 1500;
 
 bool Solver::resident_block(int nq, int md) const
@@ -43,8 +62,18 @@ Solver::ResPlan Solver::resident_plan(int nq, int md)
     const bool wide = vk == VK_C64;
     int pow = 1;
     while (pow < nq) pow *= 2;
+    if (vk == VK_C32 && !bicg && nq > 16 && mesh->nnz * (long)pow > RES_MAX_MACS) return none;
     int T = mesh->n <= RES_ONE_WG ? RES_WG : pow;
-    if ((long)T * mesh->nnz > RES_MAX_ENTRIES && T > 1 && T < RES_WG) T = std::max(1, pow / (wide ? 8 : RES_KC));
+    if (T > 1 && T < RES_WG) {
+        const int per = (mesh->n + RES_WG / T * RES_NT - 1) / (RES_WG / T * RES_NT);   // rows a thread, one column a team
+        const long xcd = std::min(T, 8) * (long)mesh->nnz;
+        bool few = (long)T * mesh->nnz > RES_MAX_ENTRIES;
+        if (cplx && per > 4) few |= bicg || xcd > RES_XCD_ENTRIES;
+        if (wide && bicg && per > 2) few |= T <= 4 || xcd > 2 * RES_XCD_ENTRIES;
+        // (BiCGSTAB, n 31,525 c32 x 17 to 32: two teams 75-76 us, four 73-75, the
+        // launch sequence 74-75)
+        if (few) T = std::max(1, pow / (wide || (bicg && pow > RES_KC) ? 8 : RES_KC));
+    }
     for (;; T /= 2) {
         if (T < 1) return none;
         const int nr = RES_WG / T;
