@@ -20,6 +20,9 @@ void launch_jacobian_nodal(Mesh &m, int nq, int nm, const double *d_dphi, int ld
 bool launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
                            int nqm, const double *d_proj, int logscale, double *d_J, int dmax, hipStream_t st, bool cw,
                            double *d_Jkap);
+// whether its operands are kept for all nodes of the mesh; for larger meshes
+// they are made in parts, on each call
+bool jacobian_tiles_whole(const Mesh &m, int dmax);
 // Element-basis Jacobian: d_J (2 nqm) x (2 elen) row-major, or with cw the
 // nqm x elen blocks d_J (mua) and d_Jkap (kappa, either may be null) from real
 // fields with zero imaginary parts and nqm real projections.  mvec_n > 0: the

@@ -369,17 +369,40 @@ void launch_real_to_cplx(long rows, int cols, const double *src, int ld, double 
     TMI_LAUNCH_CHECK();
 }
 
-// The matrix-core kernel pads the neighbours to 16 or 32.  Up to 16 it was
-// faster at every size measured (ms, per-node kernel against it: 3,169 nodes
-// 2 x 2 links 0.030 / 0.027, 32 x 32 0.092 / 0.055; 59,319 nodes 0.517 / 0.170
-// and 1.788 / 0.952).  With longer rows most of the 32 may be padding: on
-// triangulated random points (mean 7, longest 17; 40,000 nodes) 0.187 / 0.396
-// at 4 x 4 links and 1.08 / 1.49 at 32 x 32, on tetrahedra (mean 16.3, longest
-// 32; 59,887 nodes) 0.735 / 0.659 and 3.61 / 2.57, but with 2,844 nodes 0.056 /
-// 0.060 at 8 x 8 links against 0.068 / 0.064 at 16 x 16.
-static bool jacobian_tiles_pay(const Mesh &m, int nq, int nm, int dmax)
+// Whether the matrix-core kernel is the faster one: its cost follows the tiles
+// of 16 x 16 pairs, however full, and neighbours padded to 8, 16 or 32; that of
+// the per-node kernel the neighbours, the pairs (it scans all of them) and the
+// links.  In ns a node, fitted to calls with 1 x 1 to 64 x 64 sources and
+// detectors, every pair, 4 or 1 of a source's detectors linked, on disks, cylinders,
+// ellipsoids and triangulated points (per-node / matrix-core kernel in ms):
+//   n 103,267, 14.5 neighbours   1 x 1 0.858 / 0.281    16 x 16 1.227 / 0.459
+//     32 x 32 3.029 / 1.658      17 x 17, 289 links 1.510 / 1.101, 17 links 1.084 / 1.049
+//   n 30,301, 7 neighbours       2 x 2 0.120 / 0.069    32 x 32 0.700 / 0.252
+//     17 x 17, 289 links 0.247 / 0.222, 17 links 0.171 / 0.206
+//   n 287,496 (in parts, below)  1 x 1 2.604 / 1.864    16 x 16 4.038 / 2.405
+//     32 x 32, 32 links 5.407 / 4.220    17 x 17, 17 links 3.221 / 4.098
+// Below 16,384 nodes the runs are short (n 3,169: 17 x 17, 289 links 0.048 /
+// 0.049; n 8,752: 17 links 0.105 / 0.110); where the operands are made in parts on each call (above 262,144
+// nodes), that comes on top.  A single tile was the faster one everywhere.
+// Padded to 32 it costs about 3 + 7.7 a tile.  That pays for full tiles on rows
+// that are long enough:
+//   n 60,886, 16.3 neighbours, 32 at most    16 x 16 1.709 / 0.754   32 x 32
+//     3.443 / 2.571, 512 links 2.769 / 2.402, 32 links 1.907 / 2.141   40 x 40
+//     4.890 / 5.341   17 x 17 1.716 / 2.290
+//   n 3,482, 15.9 neighbours, 28 at most     16 x 16 0.100 / 0.069   32 x 32 0.184 / 0.154
+//   n 64,000, 12.6 neighbours, 19 at most    16 x 16 0.757 / 0.796   32 x 32 2.703 / 2.701
+//     17 x 17 0.854 / 2.296
+//   n 79,331, 16.1 neighbours (in parts)     16 x 16 1.655 / 2.102   32 x 32 4.083 / 4.683
+static bool jacobian_tiles_pay(const Mesh &m, int nq, int nm, int nqm, int dmax)
 {
-    return dmax <= 16 || (dmax <= 32 && (long)m.nnz >= 12L * m.n && (long)nq * nm >= 256);
+    const double d = (double)m.nnz / m.n, pairs = (double)nq * nm, tiles = (double)((nq + 15) / 16) * ((nm + 15) / 16);
+    const bool whole = jacobian_tiles_whole(m, dmax);
+    if (dmax > 16)
+        return dmax >= 24 && dmax <= 32 && d >= 15.0 && whole && (tiles == 1 ? pairs >= 192 : nqm >= 192 * tiles);
+    if (tiles == 1) return true;
+    const double node = 0.53 * d + 0.0035 * d * nm + 0.025 * nq + (0.0016 + 0.00044 * d) * pairs + 0.009 * nqm;
+    const double tile = dmax <= 8 ? 0.8 + 1.5 * tiles + 0.002 * nqm : 0.3 + 2.5 * tiles + 0.005 * nqm;
+    return tile + (m.n < 16384 ? 1.5 : 0.0) + (whole ? 0.0 : 3.5) < node;
 }
 
 void launch_jacobian_nodal(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
@@ -387,7 +410,7 @@ void launch_jacobian_nodal(Mesh &m, int nq, int nm, const double *d_dphi, int ld
                            double *d_Jkap)
 {
     if (cw && !d_J && !d_Jkap) return;
-    if (jacobian_tiles_pay(m, nq, nm, dmax) &&
+    if (jacobian_tiles_pay(m, nq, nm, nqm, dmax) &&
         launch_jacobian_tiles(m, nq, nm, d_dphi, ldd, d_aphi, lda, nqm, d_proj, logscale, d_J, dmax, st, cw, d_Jkap))
         return;
     // LDS row stride: the neighbour count rounded up to odd, so that the

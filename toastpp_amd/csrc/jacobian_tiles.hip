@@ -334,6 +334,13 @@ __global__ void __launch_bounds__(JT_NT, 3) k_jac_tiles(JtArgs A)
     }
 }
 
+// tiles of neighbours a side, and bytes of a node's operands (4 KB up to 16
+// neighbours, 16 KB up to 32)
+static int jt_of(int dmax) { return dmax <= 16 ? 1 : 2; }
+static size_t jt_node_bytes(int dmax) { return 2 * 256 * sizeof(double) * jt_of(dmax) * jt_of(dmax); }
+
+bool jacobian_tiles_whole(const Mesh &m, int dmax) { return (size_t)m.n <= JT_OPS_BYTES / jt_node_bytes(dmax); }
+
 bool launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ldd, const double *d_aphi, int lda,
                            int nqm, const double *d_proj, int logscale, double *d_J, int dmax, hipStream_t st, bool cw,
                            double *d_Jkap)
@@ -347,11 +354,10 @@ bool launch_jacobian_tiles(Mesh &m, int nq, int nm, const double *d_dphi, int ld
     a.rowptr = m.rowptr.p; a.colidx = m.colidx.p;
     a.dphi = (const double2 *)d_dphi; a.aphi = (const double2 *)d_aphi;
     a.lk = m.d_lk.p; a.proj = d_proj; a.J = d_J; a.Jkap = d_Jkap;
-    const int jt = dmax <= 16 ? 1 : 2;
-    // the operands of all nodes are kept with the mesh up to JT_OPS_BYTES (4 KB
-    // a node up to 16 neighbours); beyond, they are made for a part of the
-    // nodes at a time, on each call
-    const size_t per = 2 * 256 * (size_t)jt * jt * sizeof(double);
+    const int jt = jt_of(dmax);
+    // the operands of all nodes are kept with the mesh up to JT_OPS_BYTES;
+    // beyond, they are made for a part of the nodes at a time, on each call
+    const size_t per = jt_node_bytes(dmax);
     const int part = (int)std::min<size_t>(m.n, JT_OPS_BYTES / per);
     const bool whole = part == m.n;
     std::unique_lock<std::mutex> lock(m.jac_mu);

@@ -696,16 +696,15 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
                         p = first[j] ? r[e][j]
                                      : vadd(r[e][j], res_scale(vsub(pv[e][j], res_scale(y[e][j], om[j])), br[j]));
                     }
-                    if constexpr (M == RES_BICG) {
-                        // the stage holds s of the last iteration: an idle
-                        // column's p goes back too, for its product below
-                        if (act[j]) pv[e][j] = p;
-                        else p = pv[e][j];
+                    if (act[j]) {
+                        if constexpr (M == RES_BICG) pv[e][j] = p;
                         sp[j] = p;
-                    } else if (act[j]) {
-                        sp[j] = p;
+                        if (a.nr > 1) st_pub(pp + j, p);
+                    } else if constexpr (M == RES_BICG) {
+                        // the stage holds s of its last iteration: an idle
+                        // column's p goes back, for its product below
+                        sp[j] = pv[e][j];
                     }
-                    if (act[j] && a.nr > 1) st_pub(pp + j, p);
                 }
             }
         }
