@@ -104,6 +104,8 @@ struct ResArgs {
     const void *b;                   // caller's right-hand sides [n][ld]
     void *x;                         // caller's fields: initial guess in, solution out
     long ld;
+    int q0;                          // first column of the block in b and x: 0 (as a constant it costs other
+                                     // registers and 4 % of the c64 COCG solve, n 31,525 x 16)
     void *pub_p, *pub_s;             // published vectors [T][n][kc]
     void *x64;                       // FP64 solution [T][n][kc], published
     void *rd0;                       // shadow residual of the FP64 BiCGSTAB [T][n][kc], private to its owner
@@ -545,7 +547,7 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
     // ---- right-hand side norms, initial guess published
     CLEAR_D;
     FOR_E if (ON(e)) {
-        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + c0 + c;
+        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + a.q0 + c0 + c;
         FOR_J if (c + j < ncol) {
             const V64 b = ((const V64 *)a.b)[node + j];
             d[0][j] += dotR(b, b);
@@ -588,7 +590,7 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
             bool any = false;
             FOR_J any |= OUT(I_ACTIVE, j) != 0;
             if (any) FOR_E if (ON(e)) {
-                const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + c0 + c;
+                const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + a.q0 + c0 + c;
                 V64 s[CL];
                 S64 w[CL];
                 FOR_J { s[j] = vzero<V64>(); w[j] = MF ? (S64)omg[min(c + j, ncol - 1)] : (S64)1; }
@@ -696,14 +698,16 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
                         p = first[j] ? r[e][j]
                                      : vadd(r[e][j], res_scale(vsub(pv[e][j], res_scale(y[e][j], om[j])), br[j]));
                     }
-                    if (act[j]) {
-                        if constexpr (M == RES_BICG) pv[e][j] = p;
+                    if constexpr (M == RES_BICG) {
+                        // the stage holds s of the last iteration: an idle
+                        // column's p goes back too, for its product below
+                        if (act[j]) pv[e][j] = p;
+                        else p = pv[e][j];
+                        sp[j] = p;
+                        if (act[j] && a.nr > 1) st_pub(pp + j, p);
+                    } else if (act[j]) {
                         sp[j] = p;
                         if (a.nr > 1) st_pub(pp + j, p);
-                    } else if constexpr (M == RES_BICG) {
-                        // the stage holds s of its last iteration: an idle
-                        // column's p goes back, for its product below
-                        sp[j] = pv[e][j];
                     }
                 }
             }
@@ -828,7 +832,7 @@ __global__ void __launch_bounds__(RES_NT) k_resident(ResArgs a)
     __syncthreads();
     FRESH;
     FOR_E if (ON(e)) {
-        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + c0 + c;
+        const size_t node = (size_t)a.node[r0 + ROW(e)] * a.ld + a.q0 + c0 + c;
         FOR_J if (c + j < ncol)((V64 *)a.x)[node + j] = ld_pub((const V64 *)X + AT(e) + j);
     }
     if (rank == 0 && tid < ncol) {
