@@ -113,3 +113,31 @@ def test_few_teams_on_many_rows(solver, mode, nq):
         assert f.LastResident() == (not sequence, 0)
         X.append(dX.to_host())
     assert (np.linalg.norm(X[0] - X[1], axis=0) / np.linalg.norm(X[1], axis=0)).max() <= 20e-10
+
+
+@pytest.mark.parametrize("kind,nq", [("disk", 1), ("disk", 17), ("disk", 64), ("ellipsoid", 6), ("ellipsoid", 33),
+                                     ("ellipsoid", 57)])
+def test_small_blocks_run_resident(kind, nq):
+    """The blocks of test_resident_gpu.py run resident there, but for those
+    whose three FP64 vectors a thread cannot hold (33 and more complex columns
+    of 9,261 rows with BiCGSTAB), which it solves by the launch sequence twice."""
+    if kind == "disk":
+        (nodes, el), Q = G.disk(25.0, 22), G.ring(nq, 25.0)
+    else:
+        nodes, el = G.ellipsoid(80.0, 65.0, 90.0, 20)
+        Q = G._ellipsoid_ring_points(80.0, 65.0, 90.0, [-45.0, -15.0, 15.0, 45.0], 16, 0.0)[np.arange(nq) * 64 // nq]
+    mesh = T.Mesh(data=(nodes, el))
+    mesh.SetQM(Q, Q[:1])
+    B = np.ascontiguousarray(mesh.Qvec(width=2.0).toarray())
+    for solver, mode in (("CG", "mixed"), ("CG", "fp64_block"), ("COCG", "mixed"), ("COCG", "fp64"),
+                         ("BICGSTAB", "mixed"), ("BICGSTAB", "fp64_block")):
+        f = T.FwdSolver(mesh, solver, 1e-10, complex=solver != "CG")
+        f.SetMode(mode)
+        f.SetPrecon("DIAG")
+        f.Allocate()
+        f.Reset(T.Solution(*G.params(nodes, 7)), 100.0 * 2 * np.pi * 1e-6 if f.complex else 0.0)
+        b = np.ascontiguousarray(B if f.complex else B.real)
+        dB, dX = L.DeviceArray.from_host(b), L.DeviceArray(b.shape, b.dtype)
+        f.CalcFieldsDevice(nq, dB.ptr, dX.ptr)
+        held = not (kind == "ellipsoid" and nq >= 33 and (solver, mode) == ("BICGSTAB", "fp64_block"))
+        assert f.LastResident() == (held, 0), (solver, mode)
