@@ -328,7 +328,8 @@ int tmi_test_resident(tmi_solver s, int what);
  * 8 iterations and the reliable update when it falls due, 64 to 104 kernel
  * launches -- is captured once per workspace and operator and replayed as
  * one graph launch; 0 launches the kernels one by one.  Same kernels, same
- * arguments, same order: results are identical either way. */
+ * arguments, same order: results are identical either way.  Either call keeps
+ * the handle on the launch sequence (tmi_solver_set_tile). */
 int tmi_solver_set_graphs(tmi_solver s, int enable);
 /* Measurement hook (no reference counterpart): time `reps` launches of one
  * kernel of the last CalcFields tile with HIP events on the library stream.

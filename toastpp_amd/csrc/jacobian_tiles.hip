@@ -1,6 +1,7 @@
 // Nodal-basis Jacobian on the FP64 matrix cores: GenerateJacobian_mesh
 // (jacobian.cc:441-497) and its CW form (:727-790) for meshes whose rows hold
-// at most 32 neighbours.
+// at most 32 neighbours, where jacobian_tiles_pay (jacobian_kernels.hip) finds
+// it the faster kernel.
 //
 // Per node i and link (q, m) the PMDFs are f_q^T A_i g_m and f_q^T B_i g_m
 // over the neighbours of i (jacobian_kernels.hip states A_i and B_i).  A

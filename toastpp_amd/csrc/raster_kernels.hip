@@ -701,7 +701,10 @@ __device__ inline void grid_record(const double2 *__restrict__ v, int g, const G
 }
 
 // Records of all columns, fgs[c][s], for the gradient through G, which reads
-// each of them several times; thread per point, blocks over the columns
+// each of them several times; thread per point, blocks over the columns.  The
+// call (89,280 voxels of a 48^3 basis, 64^3 points; 2 / 16 / 32 sources) takes
+// 0.17 / 1.24 / 2.49 ms against 0.45 / 1.43 / 2.59 with maps read by rows of
+// columns and records turned through LDS; the sums through G are the rest.
 __global__ void __launch_bounds__(256) k_grid_grad(int slen, int ncols, GradDesc gd, const int *__restrict__ s2b,
                                                    const int *__restrict__ mask, long glen,
                                                    const double2 *__restrict__ fgv, double2 *__restrict__ fgs)
